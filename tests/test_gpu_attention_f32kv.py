@@ -1,0 +1,87 @@
+"""Matrix-core attention over contiguous f32 K/V at the edges of its tiles:
+head dims below, at and between the compiled ones, slot counts around 16, key
+counts around a tile and a workgroup's round of tiles, both output splits (a
+quarter of the dims per workgroup, and all of them), and non-finite V rows that
+only some query rows attend.
+
+Tolerance as in the other attention tests: 2e-5 of the largest |V| (f32 sums
+of at most 1200 products in another order, exp within an ulp) plus an ulp."""
+from __future__ import annotations
+
+import numpy as np
+import pytest
+
+import oracle
+
+pytestmark = pytest.mark.gpu
+torch = pytest.importorskip("torch")
+
+
+def _rows(q, k, v, nh, nkv, hd, ql, kvl, causal, window):
+    from fellm_amd import _lib
+
+    qd, kd, vd = (torch.from_numpy(a).cuda() for a in (q, k, v))
+    out = torch.full_like(qd, float("nan"))
+    rc = _lib.lib().fellm_rocm_attention_f32kv_rows(qd.data_ptr(), out.data_ptr(), ql, nh, nkv, hd, kd.data_ptr(),
+                                                    vd.data_ptr(), kvl, 0.0, int(causal), window,
+                                                    torch.cuda.current_stream().cuda_stream)
+    assert rc == 0, rc
+    return out.cpu().numpy()
+
+
+def _inputs(rng, nh, nkv, hd, ql, kvl):
+    return (rng.normal(size=nh * ql * hd).astype(np.float32), rng.normal(size=(kvl, nkv * hd)).astype(np.float32),
+            rng.normal(size=(kvl, nkv * hd)).astype(np.float32))
+
+
+@pytest.mark.parametrize("hd", [4, 60, 64, 68, 128, 132, 256])
+@pytest.mark.parametrize("nh,nkv,ql,kvl", [(7, 1, 1, 129), (8, 8, 3, 16), (8, 2, 300, 301), (16, 16, 70, 1100),
+                                           (8, 1, 600, 640)])
+def test_rows_edges(hd, nh, nkv, ql, kvl):
+    rng = np.random.default_rng(hd * 7 + ql)
+    q, k, v = _inputs(rng, nh, nkv, hd, ql, kvl)
+    got = _rows(q, k, v, nh, nkv, hd, ql, kvl, True, 0)
+    ref = oracle.fa2_attention(q, k, v, nh, nkv, hd, ql, kvl, float(np.float32(1 / np.sqrt(hd))), True, 0)
+    assert np.abs(got - ref).max() <= 2e-5 * np.abs(v).max() + np.abs(ref).max() * 2.0 ** -23
+
+
+@pytest.mark.parametrize("causal,window", [(True, 0), (True, 5), (False, 9)])
+@pytest.mark.parametrize("bad", [np.inf, -np.inf, np.nan])
+def test_rows_nonfinite_value_stays_with_its_rows(causal, window, bad):
+    """Rows that do not attend a key with a non-finite V get the result they
+    would have without it; rows that do get a non-finite one."""
+    nh, nkv, hd, ql, kvl = 8, 2, 64, 150, 170
+    rng = np.random.default_rng(3)
+    q, k, v = _inputs(rng, nh, nkv, hd, ql, kvl)
+    at = 100
+    v2 = v.copy()
+    v2[at, 5] = bad  # dim 5 of KV head 0
+    clean = _rows(q, k, v, nh, nkv, hd, ql, kvl, causal, window).reshape(nh, ql, hd)
+    got = _rows(q, k, v2, nh, nkv, hd, ql, kvl, causal, window).reshape(nh, ql, hd)
+    row = np.arange(ql)
+    last = kvl - ql + row
+    sees = ((at <= last) & ((window == 0) | (at > last - window))) if causal else np.abs(row - at) < window
+    hit = np.zeros((nh, ql, hd), bool)
+    hit[:nh // nkv, :, 5] = sees[None, :]
+    assert np.all(~np.isfinite(got[hit]))
+    assert np.abs(got[~hit] - clean[~hit]).max() <= 2e-5 * np.abs(v).max()
+
+
+@pytest.mark.parametrize("rows,past", [(16, 1), (33, 47), (80, 1000)])
+def test_canvas_edges(rows, past):
+    from fellm_amd import _lib
+
+    nh, nkv, hd = 16, 4, 128
+    rng = np.random.default_rng(rows + past)
+    q = rng.normal(size=(rows, nh * hd)).astype(np.float32)
+    k, v = (rng.normal(size=(past, nkv * hd)).astype(np.float32) for _ in range(2))
+    ck, cv = (rng.normal(size=(rows, nkv * hd)).astype(np.float32) for _ in range(2))
+    d = [torch.from_numpy(a).cuda() for a in (q, k, v, ck, cv)]
+    out = torch.full_like(d[0], float("nan"))
+    rc = _lib.lib().fellm_rocm_attention_f32kv(d[0].data_ptr(), out.data_ptr(), rows, nh, nkv, hd, d[1].data_ptr(),
+                                               d[2].data_ptr(), 0, past, d[3].data_ptr(), d[4].data_ptr(), rows, 0.0,
+                                               torch.cuda.current_stream().cuda_stream)
+    assert rc == 0, rc
+    ref = oracle.attention_f32kv(q, nh, nkv, hd, k, v, 0, past, ck, cv, rows)
+    assert np.abs(out.cpu().numpy() - ref).max() <= 2e-5 * max(np.abs(v).max(), np.abs(cv).max()) + \
+        np.abs(ref).max() * 2.0 ** -23

@@ -10,25 +10,42 @@
 //   :3394-3446) is fed; K/V rows as crates/fellm-plugin-abi/src/paged_ctx.rs
 //   :138-174 address them.
 //
-// Work split.  One wavefront per (batch row b, KV head g, key split s); the
-// G = n_heads / n_kv query heads that share KV head g are processed together,
-// so every K/V byte is read once.  Keys go in cache blocks of 16 tokens:
-//  * Q.K^T on the matrix cores: v_mfma_f32_16x16x16f16 with A = the block's K
-//    rows (16 tokens x 16 dims per step) and B = q^T (16 dims x 16 head slots).
-//    q is split into f16 high and low parts (two MFMAs per step), so the
-//    products with the f16 cache are exact and the f32 accumulation carries
-//    q to ~2^-22 relative; a bf16 cache uses bf16 MFMAs with a three-way split.
-//    The contraction order over dims is a permutation shared by A and B: lane
-//    group i = lane / 16 holds dims 32(s/2) + 8i + 4(s%2) .. +3 of step s.
-//  * Online softmax in f32 per head (block max across the 64 lanes, exp,
-//    rescale by exp(m_old - m_new)), probabilities exchanged through LDS.
-//  * P.V on the vector ALUs: lane (token group tg = lane / 16, dim slice
-//    ds = lane % 16) accumulates HD/16 dims of all G heads over tokens
-//    4i + tg, in f32; the four token groups are summed at the end.
-// Splits (several wavefronts per (b, g) when b * n_kv is small) write
-// unnormalised partial sums with their running max and denominator; a second
-// kernel combines them.  Tokens outside [lo, seq) are masked with -inf and
-// their V rows read as zero, so stale cache bytes never reach the output.
+// Work split.  One workgroup per (key split s, batch row b, KV head g), its
+// four wavefronts taking every fourth pair of cache blocks and merging their
+// (max, sum, accumulators) through LDS at the end; the
+// G = n_heads / n_kv query heads that share KV head g are processed together
+// (as up to 16 head slots), so every K/V byte is read once.  Both products of a
+// pair of blocks (2 x 16 tokens) run on the matrix cores:
+//  * S^T = K . Q^T by v_mfma_f32_16x16x32: A = a block's K rows (lane = token
+//    lane % 16, dims 32c + 8 (lane / 16) .. +7 of step c), B = q.  q is split
+//    into f16 high and low parts (two MFMAs per step), so the products with
+//    the f16 cache are exact and the f32 accumulation carries q to ~2^-22
+//    relative; a bf16 cache uses bf16 MFMAs with a three-way split.
+//  * Lane (head slot lane % 16, group lane / 16) then owns the scores of
+//    tokens 4 group .. +3 of each block, which is the layout the second
+//    product takes its B operand in, so the online softmax runs in f32 with
+//    its maximum, rescaling factor and sum per lane, and nothing goes through
+//    LDS.
+//  * out^T = V^T . P^T: the probabilities split as q is (f16 parts after a
+//    scaling by 2^14, so that small ones keep their bits: two parts hold p to
+//    2^-24 relative, three bf16 parts the same), A = V^T assembled from the
+//    lanes' row pieces by byte permutes, f32 accumulation.  The lower parts of
+//    q and p are summed apart from the first, which costs nothing and takes
+//    the error against 64 bits from 0.9 .. 1.15 times that of f32 sums on the
+//    vector ALUs to 0.55 .. 1.05 times.
+// The next pair's K is requested once Q.K has read the registers, its V once
+// P.V has.
+//
+// Bound by the cache's bytes.  Against the kernel before it (one wavefront per
+// workgroup, P.V on the vector ALUs, two blocks ahead): 256 rows of 256 .. 4096
+// keys, 64/8 heads of 128, bf16 (2.39 GB) 629 -> 414 us; the same of 4096 keys
+// each 747 -> 709 (6.1 TB/s); one row of 32768 keys, 32/8 heads, f16 33.9 -> 27.3.
+//
+// Splits write unnormalised partial sums with their running max and
+// denominator; a second kernel combines them.  A row whose keys fit one split
+// is finished by that split and skipped by the combine.  Tokens outside
+// [lo, seq) are masked with -inf and their V rows read as zero, so stale
+// cache bytes never reach the output.
 #include "common.hpp"
 
 #include "fellm_rocm.h"
@@ -36,8 +53,8 @@
 namespace fellm {
 namespace {
 
-typedef _Float16 half4_t __attribute__((ext_vector_type(4)));
-typedef short short4_t __attribute__((ext_vector_type(4)));
+typedef _Float16 half8_t __attribute__((ext_vector_type(8)));
+typedef __bf16 bf8_t __attribute__((ext_vector_type(8)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
@@ -47,6 +64,16 @@ constexpr uint32_t kBlockTokens = 16;  // tokens per cache block handled by one 
 // A split's partial record per head slot: HD sums, m, l and two unused
 // floats, so that every record starts on a 16-byte boundary.
 constexpr uint32_t kRecTail = 4;
+// Wavefronts that share a split's blocks.  Measured (kernels of 1 / 2 / 4 / 8,
+// f16): 256 rows of 256 .. 4096 keys 445 / 416 / 396 / 462 us, one row of 32768
+// keys 31.6 / 26.3 / 27.3 / 31.0, 256 rows of 16 .. 256 keys 36 / 30 / 36 / 67.
+constexpr uint32_t kDecodeWaves = 4;
+// Cache policies of the K and V reads.  V is read once by whole lines, so it
+// bypasses cache retention.  A K load instruction takes 64 bytes of each of
+// 16 rows, half a line, and the next one the other half: non-temporal K reads
+// fetched lines twice.  Measured (K, V non-temporal or not): 256 rows x 4096
+// keys 677 us (V only), 724 (both), 733 (K only), 737 (neither).
+constexpr int kKPolicy = 0, kVPolicy = 2;
 
 struct PagedGeom {
     const uint8_t *arena;
@@ -58,349 +85,344 @@ struct PagedGeom {
     uint32_t stride;  // elements per token row (n_kv * head_dim)
 };
 
-// Cache element policies: MFMA operand split of q and widening of V.
+// Cache element policies: the matrix-core type and the splitting of an f32
+// operand into kParts of them.
 struct CacheF16 {
     static constexpr int kParts = 2;
-    using Op = half4_t;
-    __device__ static Op part(const float (&v)[4], int p, float (&rem)[4]) {
-        Op o;
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            const _Float16 h = (_Float16)rem[e];
-            o[e] = h;
-            rem[e] = rem[e] - (float)h;
-        }
-        (void)v;
-        (void)p;
-        return o;
+    static constexpr float kPScale = 16384.0f;  // probabilities times this are split
+    // Two values rounded to nearest even and packed; the remainders replace them.
+    __device__ static uint32_t part(float &x, float &y) {
+        typedef _Float16 half2_t __attribute__((ext_vector_type(2)));
+        half2_t h;
+        h[0] = (_Float16)x;
+        h[1] = (_Float16)y;
+        x = x - (float)h[0];
+        y = y - (float)h[1];
+        return __builtin_bit_cast(uint32_t, h);
     }
-    __device__ static Op from_bits(uint32_t lo, uint32_t hi) {
-        Op o;
-        o[0] = __builtin_bit_cast(_Float16, (uint16_t)(lo & 0xffffu));
-        o[1] = __builtin_bit_cast(_Float16, (uint16_t)(lo >> 16));
-        o[2] = __builtin_bit_cast(_Float16, (uint16_t)(hi & 0xffffu));
-        o[3] = __builtin_bit_cast(_Float16, (uint16_t)(hi >> 16));
-        return o;
+    __device__ static f32x4 mfma(u32x4 a, u32x4 b, f32x4 c) {
+        return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(half8_t, a), __builtin_bit_cast(half8_t, b), c, 0,
+                                                      0, 0);
     }
-    __device__ static f32x4 mfma(Op a, Op b, f32x4 c) { return __builtin_amdgcn_mfma_f32_16x16x16f16(a, b, c, 0, 0, 0); }
-    __device__ static float widen(uint32_t bits16) { return (float)__builtin_bit_cast(_Float16, (uint16_t)bits16); }
 };
 
 struct CacheBF16 {
     static constexpr int kParts = 3;
-    using Op = short4_t;
-    __device__ static Op part(const float (&v)[4], int p, float (&rem)[4]) {
-        Op o;
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            // round to nearest even bf16, keep the remainder for the next part
-            const uint32_t u = __float_as_uint(rem[e]);
-            const uint32_t r = (u + 0x7fffu + ((u >> 16) & 1u)) & 0xffff0000u;
-            o[e] = (short)(r >> 16);
-            rem[e] = rem[e] - __uint_as_float(r);
-        }
-        (void)v;
-        (void)p;
-        return o;
+    static constexpr float kPScale = 1.0f;
+    __device__ static uint32_t part(float &x, float &y) {
+        typedef __bf16 bf2_t __attribute__((ext_vector_type(2)));
+        bf2_t h;
+        h[0] = (__bf16)x;
+        h[1] = (__bf16)y;
+        const uint32_t u = __builtin_bit_cast(uint32_t, h);
+        x = x - __uint_as_float(u << 16);
+        y = y - __uint_as_float(u & 0xffff0000u);
+        return u;
     }
-    __device__ static Op from_bits(uint32_t lo, uint32_t hi) {
-        Op o;
-        o[0] = (short)(lo & 0xffffu);
-        o[1] = (short)(lo >> 16);
-        o[2] = (short)(hi & 0xffffu);
-        o[3] = (short)(hi >> 16);
-        return o;
+    __device__ static f32x4 mfma(u32x4 a, u32x4 b, f32x4 c) {
+        return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf8_t, a), __builtin_bit_cast(bf8_t, b), c, 0, 0,
+                                                       0);
     }
-    __device__ static f32x4 mfma(Op a, Op b, f32x4 c) {
-        return __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, b, c, 0, 0, 0);
-    }
-    __device__ static float widen(uint32_t bits16) { return __uint_as_float(bits16 << 16); }
 };
 
-// Keys of split s for a row of length seq: blocks [b0, b1) of the range
-// [lo, seq) (lo > 0 only for a causal window), in chunks of bps blocks.
-__device__ __forceinline__ void split_range(uint32_t seq, uint32_t lo, uint32_t s, uint32_t bps, uint32_t &b0,
-                                            uint32_t &b1) {
-    const uint32_t first = lo / kBlockTokens, last = (seq + kBlockTokens - 1) / kBlockTokens;
-    b0 = first + s * bps;
-    b1 = b0 + bps < last ? b0 + bps : last;
-    if (b0 > last) b0 = last;
+// v[0..7] as kParts operands.
+template <typename C>
+__device__ __forceinline__ void split8(const float (&v)[8], u32x4 (&o)[C::kParts]) {
+    float rem[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) rem[i] = v[i];
+#pragma unroll
+    for (int p = 0; p < C::kParts; ++p)
+#pragma unroll
+        for (int w = 0; w < 4; ++w) o[p][w] = C::part(rem[2 * w], rem[2 * w + 1]);
+}
+
+// Keys [lo, seq) of a row: cache blocks [first, last) and how many of the
+// launch's splits of bps blocks hold any.
+struct RowKeys {
+    uint32_t lo, seq, first, last, splits;
+};
+__device__ __forceinline__ RowKeys row_keys(uint32_t seq, uint32_t causal, uint32_t window, uint32_t bps,
+                                            uint32_t splits) {
+    RowKeys r;
+    r.seq = seq;
+    r.lo = (causal && window && seq > window) ? seq - window : 0;
+    r.first = r.lo / kBlockTokens;
+    r.last = (seq + kBlockTokens - 1) / kBlockTokens;
+    r.splits = (r.last - r.first + bps - 1) / bps;
+    if (r.splits > splits) r.splits = splits;  // a length past max_seq
+    return r;
+}
+
+// Maximum over the four 16-lane rows; every lane gets the result.
+__device__ __forceinline__ float rows_max(float v) {
+    const uint32_t u = __float_as_uint(v);
+    const auto a = __builtin_amdgcn_permlane32_swap(u, u, false, false);
+    v = fmaxf(__uint_as_float(a[0]), __uint_as_float(a[1]));
+    const uint32_t w = __float_as_uint(v);
+    const auto b = __builtin_amdgcn_permlane16_swap(w, w, false, false);
+    return fmaxf(__uint_as_float(b[0]), __uint_as_float(b[1]));
 }
 
 // Q: query activation policy, O: output policy, C: cache policy, HD: head
-// dim (64, 128 or 256), GM: maximum query heads per KV head (8 or 16).
-template <typename Q, typename O, typename C, int HD, int GM, int DEPTH>
-__global__ __launch_bounds__(kWave) void paged_decode_kernel(const typename Q::T *__restrict__ q,
+// dim (64, 128 or 256).  rec_heads: head slots of a partial record.  early:
+// the first blocks are requested before the row length is known.
+template <typename Q, typename O, typename C, int HD>
+__global__ __launch_bounds__(kWave * kDecodeWaves) void paged_decode_kernel(const typename Q::T *__restrict__ q,
                                                              typename O::T *__restrict__ out,
                                                              float *__restrict__ part, const uint32_t *__restrict__ lens,
-                                                             const uint32_t *__restrict__ table, PagedGeom geo,
-                                                             uint32_t n_heads, uint32_t n_kv, float scale,
-                                                             uint32_t causal, uint32_t window, uint32_t splits,
-                                                             uint32_t bps) {
-    constexpr int NS = HD / 16;  // MFMA k-steps
-    constexpr int NKL = HD / 32; // 16-byte K loads per lane per block
-    constexpr int DP = HD / 16;  // dims per lane in P.V
-    __shared__ __align__(16) float lds_p[kBlockTokens * 16];
-    __shared__ __align__(16) float lds_h[16];
+                                                             PagedGeom geo, uint32_t batch, uint32_t n_heads,
+                                                             uint32_t n_kv, float scale, uint32_t causal,
+                                                             uint32_t window, uint32_t splits, uint32_t bps,
+                                                             uint32_t rec_heads, uint32_t early) {
+    constexpr int NC = HD / 32;               // Q.K steps, and 16-byte K loads per lane and block
+    constexpr int DP = HD < 128 ? 4 : 8;      // consecutive dims of a lane's V piece
+    constexpr int VH = HD / 16 / DP;          // V pieces per token row
+    constexpr int NT = HD / 16;               // output tiles
+    constexpr float kUnscale = 1.0f / C::kPScale;
 
-    const uint32_t lane = threadIdx.x;
-    const uint32_t col = lane % 16, grp = lane / 16;  // MFMA column (head slot) / lane group
-    const uint32_t s = blockIdx.x % splits;
-    const uint32_t bg = blockIdx.x / splits;
+    extern __shared__ __align__(16) float merge_lds[];
+    const uint32_t lane = threadIdx.x % kWave, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+    const uint32_t col = lane % 16, grp = lane / 16;
+    // Splits in the outer order: the later ones, which fewer rows reach, come last.
+    const uint32_t bg = blockIdx.x % (batch * n_kv), s = blockIdx.x / (batch * n_kv);
     const uint32_t g = bg % n_kv, b = bg / n_kv;
     const uint32_t G = n_heads / n_kv;
-    const size_t row_bytes = (size_t)geo.stride * 2;
+    const uint32_t row_bytes = geo.stride * 2;
     const size_t table_base = ((size_t)b * geo.n_layers + geo.layer) * geo.n_logical;
-    // One cache block's K and V slices for this lane, fetched through a
-    // buffer resource spanning the block: an absent or out-of-range block has
-    // range 0 and reads as zeros without memory traffic, so the next block is
-    // requested unconditionally while the current one is reduced.
-    struct BlockRegs {
-        uint4 kr[NKL];         // K: token col, dims 32c + 8 grp .. +7 of load c
-        uint32_t vr[4][DP / 2]; // V: token 4i + grp, dims col*DP .. +DP-1
-        bool ok;
-    };
-    auto fetch = [&](uint32_t blk, uint32_t lim, BlockRegs &R) {
+
+    // This wavefront's pairs of blocks: first + 2 (wave + kDecodeWaves n), n =
+    // 0, 1, ..  Lane l holds the physical block (~0: none, or at or past lim)
+    // of block l % 2 of pair tab0 + l / 2; a walk of more than 32 pairs reloads.
+    uint32_t tab = ~0u, tab0 = 0;
+    auto pair_block = [&](uint32_t first, uint32_t n) { return first + 2 * (wave + kDecodeWaves * n); };
+    auto load_table = [&](uint32_t first, uint32_t n, uint32_t lim) {
+        tab0 = n;
+        const uint32_t blk = pair_block(first, n + lane / 2) + lane % 2;
         const size_t ti = table_base + blk;
-        const uint64_t phys =
-            (blk < lim && blk < geo.n_logical && ti < geo.n_table) ? (uint64_t)table[ti] : ~0ull;
-        const bool ok = phys != ~0ull && (phys + 1) * geo.block_bytes <= geo.arena_len;
-        const uint8_t *base = geo.arena + (ok ? phys * geo.block_bytes : 0);
-        const Rsrc rs = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t *>(base), 0,
-                                                          ok ? (int)geo.block_bytes : 0, 0x00020000);
-        const uint32_t koff = g * HD * 2 + col * (uint32_t)row_bytes + 16 * grp;
-#pragma unroll
-        for (int c = 0; c < NKL; ++c) {
-            const u32x4 t = __builtin_amdgcn_raw_buffer_load_b128(rs, koff + 64 * c, 0, 2);
-            R.kr[c] = make_uint4(t.x, t.y, t.z, t.w);
+        tab = ~0u;
+        if (blk < lim && blk < geo.n_logical && ti < geo.n_table) {
+            const uint64_t p = geo.table[ti];
+            if ((p + 1) * geo.block_bytes <= geo.arena_len) tab = (uint32_t)p;
         }
-        const uint32_t voff = geo.block_size * (uint32_t)row_bytes + g * HD * 2 + col * DP * 2;
+    };
+    // Both blocks are read through buffer resources that span a block: an
+    // absent one has range 0 and reads as zeros without memory traffic.
+    struct Pair {
+        Rsrc rs[2];
+        bool ok[2];
+    };
+    auto pair_at = [&](uint32_t n) -> Pair {
+        Pair r;
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const uint32_t o = voff + (4 * i + grp) * (uint32_t)row_bytes;
-            if constexpr (DP == 4) {  // 8 bytes per lane
-                const u32x2 t = __builtin_amdgcn_raw_buffer_load_b64(rs, o, 0, 2);
-                R.vr[i][0] = t.x;
-                R.vr[i][1] = t.y;
-            } else {  // 16 or 32 bytes per lane
+        for (int u = 0; u < 2; ++u) {
+            const uint32_t phys = (uint32_t)__builtin_amdgcn_readlane((int)tab, (int)(2 * (n - tab0) + u));
+            r.ok[u] = phys != ~0u;
+            const uint8_t *base = geo.arena + (r.ok[u] ? phys * geo.block_bytes : 0);
+            r.rs[u] = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t *>(base), 0,
+                                                        r.ok[u] ? (int)geo.block_bytes : 0, 0x00020000);
+        }
+        return r;
+    };
+    u32x4 kr[2][NC];  // K: token col, dims 32c + 8 grp .. +7
+    auto load_k = [&](const Pair &r) {
+        const uint32_t off = g * HD * 2 + col * row_bytes + 16 * grp;
 #pragma unroll
-                for (int w = 0; w < DP / 2; w += 4) {
-                    const u32x4 t = __builtin_amdgcn_raw_buffer_load_b128(rs, o + 4 * w, 0, 2);
-                    R.vr[i][w] = t.x;
-                    R.vr[i][w + 1] = t.y;
-                    R.vr[i][w + 2] = t.z;
-                    R.vr[i][w + 3] = t.w;
+        for (int u = 0; u < 2; ++u)
+#pragma unroll
+            for (int c = 0; c < NC; ++c) kr[u][c] = __builtin_amdgcn_raw_buffer_load_b128(r.rs[u], off + 64 * c, 0, kKPolicy);
+    };
+    uint32_t vr[8][VH][DP / 2];  // V: token 4 grp + i % 4 of block i / 4, dims 128h + DP col .. +DP-1
+    auto load_v = [&](const Pair &r) {
+#pragma unroll
+        for (int i = 0; i < 8; ++i)
+#pragma unroll
+            for (int h = 0; h < VH; ++h) {
+                const uint32_t o = (geo.block_size + 4 * grp + i % 4) * row_bytes + (g * HD + 128 * h + DP * col) * 2;
+                if constexpr (DP == 4) {
+                    const u32x2 t = __builtin_amdgcn_raw_buffer_load_b64(r.rs[i / 4], o, 0, kVPolicy);
+                    vr[i][h][0] = t.x;
+                    vr[i][h][1] = t.y;
+                } else {
+                    const u32x4 t = __builtin_amdgcn_raw_buffer_load_b128(r.rs[i / 4], o, 0, kVPolicy);
+#pragma unroll
+                    for (int w = 0; w < 4; ++w) vr[i][h][w] = t[w];
                 }
             }
-        }
-        R.ok = ok;
     };
-    // Without a sliding window the split's first block is s * bps whatever
-    // the sequence length, so it is requested before the length arrives
-    // (tokens past the length are masked in process); with a window the
-    // first block depends on the length and is fetched once it is known.
-    const bool spec = !(causal && window);
-    // DEPTH blocks are in flight ahead of the one being reduced.
-    BlockRegs ra, rb, rc;
-    if constexpr (DEPTH == 2) fetch(s * bps + 1, spec ? s * bps + bps : 0u, rb);
-    fetch(s * bps, spec ? s * bps + bps : 0u, ra);
-    const uint32_t seq = lens[b];
-    const uint32_t lo = (causal && window && seq > window) ? seq - window : 0;
-    uint32_t blk0, blk1;
-    split_range(seq, lo, s, bps, blk0, blk1);
 
-    // q^T as the B operand: head slot col (= query head g*G + col), dims of step st.
-    typename C::Op qb[NS][C::kParts];
+    // Without a sliding window the split's first block is s * bps whatever
+    // the row length; `early` requests it before the length arrives (tokens
+    // past the length are masked), which a launch of few wavefronts gains
+    // from and one of many does not need.
+    Pair cur;
+    if (early) {
+        load_table(s * bps, 0, s * bps + bps);
+        cur = pair_at(0);
+        load_k(cur);
+        load_v(cur);
+    }
+    const RowKeys row = row_keys(lens[b], causal, window, bps, splits);
+    if (s >= (row.splits ? row.splits : 1)) return;
+    const uint32_t blk0 = row.first + s * bps;
+    const uint32_t blk1 = blk0 + bps < row.last ? blk0 + bps : row.last;
+    if (!early) {
+        load_table(blk0, 0, blk1);
+        cur = pair_at(0);
+        load_k(cur);
+        load_v(cur);
+    }
+
+    // q as the B operand: head slot col (= query head g*G + col), dims 32c + 8 grp .. +7
+    u32x4 qb[NC][C::kParts];
     {
-        // Steps 2j and 2j+1 use dims 32j + 8 grp .. +7: one vector load each.
         const bool hv = col < G;
         const typename Q::T *qh = q + ((size_t)b * n_heads + (size_t)g * G + (hv ? col : 0)) * HD;
-        float qv[NS / 2][8];
 #pragma unroll
-        for (int j = 0; j < NS / 2; ++j) {
-            load_f32<Q, 8>(qh + 32 * j + 8 * grp, qv[j]);
+        for (int c = 0; c < NC; ++c) {
+            float v[8];
+            load_f32<Q, 8>(qh + 32 * c + 8 * grp, v);
             if (!hv)
 #pragma unroll
-                for (int e = 0; e < 8; ++e) qv[j][e] = 0.0f;
-        }
-#pragma unroll
-        for (int st = 0; st < NS; ++st) {
-            float v[4], rem[4];
-#pragma unroll
-            for (int e = 0; e < 4; ++e) rem[e] = v[e] = qv[st / 2][4 * (st % 2) + e];
-#pragma unroll
-            for (int p = 0; p < C::kParts; ++p) qb[st][p] = C::part(v, p, rem);
+                for (int e = 0; e < 8; ++e) v[e] = 0.0f;
+            split8<C>(v, qb[c]);
         }
     }
 
-    float acc[GM][DP];
+    f32x4 acc[NT];  // tile (h, j) of lane (col, grp): dims 128h + DP (4 grp + e) + j of head slot col
 #pragma unroll
-    for (int h = 0; h < GM; ++h)
-#pragma unroll
-        for (int d = 0; d < DP; ++d) acc[h][d] = 0.0f;
-    float m = -__builtin_inff(), l = 0.0f;  // running max / denominator of head slot col
+    for (int n = 0; n < NT; ++n) acc[n] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+    float m = -__builtin_inff(), l = 0.0f;  // running max, this lane's part of the denominator
 
-    auto process = [&](uint32_t blk, const BlockRegs &R) {
-        const bool blk_ok = R.ok;
-        const uint4(&kr)[NKL] = R.kr;
-        const uint32_t(&vr)[4][DP / 2] = R.vr;
-        const uint32_t t0 = blk * kBlockTokens;
-        // S^T[token 4 grp + e][head slot col]
-        f32x4 sacc = {0.0f, 0.0f, 0.0f, 0.0f};
+    for (uint32_t n = 0; pair_block(blk0, n) < blk1; ++n) {
+        // S^T[token 4 grp + e][head slot col] of both blocks
+        f32x4 sc[2], sl[2];
 #pragma unroll
-        for (int st = 0; st < NS; ++st) {
-            const uint4 &k4 = kr[st / 2];
-            const typename C::Op a = (st % 2) ? C::from_bits(k4.z, k4.w) : C::from_bits(k4.x, k4.y);
+        for (int u = 0; u < 2; ++u) sc[u] = sl[u] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
-            for (int p = 0; p < C::kParts; ++p) sacc = C::mfma(a, qb[st][p], sacc);
-        }
-        float sc[4];
-        float bmax = -__builtin_inff();
+        for (int c = 0; c < NC; ++c)
 #pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            const uint32_t t = t0 + 4 * grp + e;
-            const bool valid = blk_ok && t >= lo && t < seq;
-            sc[e] = valid ? sacc[e] * scale : -__builtin_inff();
-            bmax = fmaxf(bmax, sc[e]);
-        }
-        bmax = fmaxf(bmax, __shfl_xor(bmax, 16, kWave));
-        bmax = fmaxf(bmax, __shfl_xor(bmax, 32, kWave));
-        const float m_new = fmaxf(m, bmax);
-        const float alpha = (m > -__builtin_inff()) ? __expf(m - m_new) : 0.0f;
-        float psum = 0.0f;
+            for (int p = 0; p < C::kParts; ++p)
 #pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            const float p = sc[e] > -__builtin_inff() ? __expf(sc[e] - m_new) : 0.0f;
-            lds_p[(4 * grp + e) * 16 + col] = p;
-            psum += p;
-        }
-        psum += __shfl_xor(psum, 16, kWave);
-        psum += __shfl_xor(psum, 32, kWave);
-        // a head with no valid key yet keeps m = -inf, l = 0, alpha = 0
-        if (m_new > -__builtin_inff()) {
-            l = l * alpha + psum;
-            m = m_new;
-        }
-        if (grp == 0) lds_h[col] = m_new > -__builtin_inff() ? alpha : 1.0f;
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront", "local");
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront", "local");
-
-        float al[GM];
-#pragma unroll
-        for (int h = 0; h < GM; h += 4) {
-            const float4 t = *reinterpret_cast<const float4 *>(&lds_h[h]);
-            al[h] = t.x;
-            al[h + 1] = t.y;
-            al[h + 2] = t.z;
-            al[h + 3] = t.w;
-        }
-#pragma unroll
-        for (int h = 0; h < GM; ++h)
-#pragma unroll
-            for (int d = 0; d < DP; ++d) acc[h][d] *= al[h];
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const uint32_t t = 4 * i + grp;
-            const bool tv = blk_ok && t0 + t >= lo && t0 + t < seq;
-            float v[DP];
-#pragma unroll
-            for (int w = 0; w < DP / 2; ++w) {
-                v[2 * w] = tv ? C::widen(vr[i][w] & 0xffffu) : 0.0f;
-                v[2 * w + 1] = tv ? C::widen(vr[i][w] >> 16) : 0.0f;
-            }
-            float p[GM];
-#pragma unroll
-            for (int h = 0; h < GM; h += 4) {
-                const float4 t4 = *reinterpret_cast<const float4 *>(&lds_p[t * 16 + h]);
-                p[h] = t4.x;
-                p[h + 1] = t4.y;
-                p[h + 2] = t4.z;
-                p[h + 3] = t4.w;
-            }
-#pragma unroll
-            for (int h = 0; h < GM; ++h)
-#pragma unroll
-                for (int d = 0; d < DP; ++d) acc[h][d] = __builtin_fmaf(p[h], v[d], acc[h][d]);
-        }
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront", "local");
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront", "local");
-        };
-    if constexpr (DEPTH == 2) {
-        if (!spec) {
-            fetch(blk0, blk1, ra);
-            fetch(blk0 + 1, blk1, rb);
-        }
-        for (uint32_t blk = blk0; blk < blk1; blk += 3) {
-            fetch(blk + 2, blk1, rc);
-            process(blk, ra);
-            if (blk + 1 >= blk1) break;
-            fetch(blk + 3, blk1, ra);
-            process(blk + 1, rb);
-            if (blk + 2 >= blk1) break;
-            fetch(blk + 4, blk1, rb);
-            process(blk + 2, rc);
-        }
-    } else {
-        if (!spec) fetch(blk0, blk1, ra);
-        for (uint32_t blk = blk0; blk < blk1; blk += 2) {
-            fetch(blk + 1, blk1, rb);
-            process(blk, ra);
-            if (blk + 1 >= blk1) break;
-            fetch(blk + 2, blk1, ra);
-            process(blk + 1, rb);
-        }
-    }
-
-    // Sum the four token groups; lanes 0..15 then hold dims col*DP .. of every head.
-#pragma unroll
-    for (int h = 0; h < GM; ++h)
-#pragma unroll
-        for (int d = 0; d < DP; ++d) {
-            acc[h][d] += __shfl_xor(acc[h][d], 16, kWave);
-            acc[h][d] += __shfl_xor(acc[h][d], 32, kWave);
-        }
-    if (grp == 0) lds_h[col] = l;
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront", "local");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront", "local");
-    // The epilogue loops over head slots are unrolled (with a guard rather
-    // than a break: a loop with a second exit is not fully unrolled at GM 16,
-    // and acc then lives in scratch), except where acc (GM x HD / 16 floats
-    // per lane) cannot stay in registers anyway: at 16 x 256 unrolling only
-    // multiplies the compile time.
-    constexpr int kEpiUnroll = GM * DP > 128 ? 1 : GM;
-    if (splits == 1) {
-        if (grp == 0) {
-#pragma unroll kEpiUnroll
-            for (int h = 0; h < GM; ++h) {
-                if ((uint32_t)h < G) {
-                    const float lh = lds_h[h];
-                    const float inv = lh > 0.0f ? 1.0f / lh : 0.0f;
-                    typename O::T *o = out + ((size_t)b * n_heads + (size_t)g * G + h) * HD + col * DP;
-                    float r[DP];
-#pragma unroll
-                    for (int d = 0; d < DP; ++d) r[d] = lh > 0.0f ? acc[h][d] * inv : 0.0f;
-                    store_f32<O, DP>(o, r);
+                for (int u = 0; u < 2; ++u) {
+                    // the parts below the first in a sum of their own
+                    f32x4 &d = p ? sl[u] : sc[u];
+                    d = C::mfma(kr[u][c], qb[c][p], d);
                 }
+        if (n + 1 - tab0 == (uint32_t)kWave / 2) load_table(blk0, n + 1, blk1);
+        const Pair next = pair_at(n + 1);
+        __builtin_amdgcn_sched_barrier(0);  // a second register set of K would cost occupancy
+        load_k(next);
+
+        const uint32_t t0 = pair_block(blk0, n) * kBlockTokens;
+        const bool edge = t0 < row.lo || t0 + 2 * kBlockTokens > row.seq || !cur.ok[0] || !cur.ok[1];
+        float p[8], mx = -__builtin_inff();
+#pragma unroll
+        for (int i = 0; i < 8; ++i) p[i] = (sc[i / 4][i % 4] + sl[i / 4][i % 4]) * scale;
+        if (edge) {
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {
+                const uint32_t t = t0 + (i / 4) * kBlockTokens + 4 * grp + i % 4;
+                const bool on = cur.ok[i / 4] && t >= row.lo && t < row.seq;
+                if (!on) p[i] = -__builtin_inff();
+#pragma unroll
+                for (int h = 0; h < VH; ++h)
+#pragma unroll
+                    for (int w = 0; w < DP / 2; ++w) vr[i][h][w] = on ? vr[i][h][w] : 0u;
             }
         }
+#pragma unroll
+        for (int i = 0; i < 8; ++i) mx = fmaxf(mx, p[i]);
+        const float mn = fmaxf(m, rows_max(mx));
+        if (__any(mn > m)) {  // most pairs raise no head's maximum
+            const float alpha = m > -__builtin_inff() ? __expf(m - mn) : 0.0f;
+            l *= alpha;
+#pragma unroll
+            for (int n = 0; n < NT; ++n) acc[n] *= alpha;
+            m = mn;
+        }
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            p[i] = p[i] > -__builtin_inff() ? __expf(p[i] - m) : 0.0f;
+            l += p[i];
+            p[i] *= C::kPScale;
+        }
+        u32x4 pb[C::kParts];
+        split8<C>(p, pb);
+#pragma unroll
+        for (int h = 0; h < VH; ++h)
+#pragma unroll
+            for (int j = 0; j < DP; ++j) {
+                u32x4 a;  // dim DP col + j of the eight tokens
+#pragma unroll
+                for (int w = 0; w < 4; ++w)
+                    a[w] = __builtin_amdgcn_perm(vr[2 * w + 1][h][j / 2], vr[2 * w][h][j / 2],
+                                                 j % 2 ? 0x07060302u : 0x05040100u);
+                // the pair's sum by itself, smallest part first, then once onto the running one
+                f32x4 t = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+                for (int x = C::kParts - 1; x >= 0; --x) t = C::mfma(a, pb[x], t);
+                acc[h * DP + j] += t;
+            }
+        __builtin_amdgcn_sched_barrier(0);
+        load_v(next);
+        cur = next;
+    }
+    l += __shfl_xor(l, 16, kWave);
+    l += __shfl_xor(l, 32, kWave);
+
+    // Merge the wavefronts pairwise through LDS: [half, 2 half) hand theirs to [0, half).
+    constexpr uint32_t kMerge = (NT * 4 + 2) * kWave;  // floats per wavefront
+#pragma unroll
+    for (uint32_t half = kDecodeWaves / 2; half > 0; half /= 2) {
+        float *rec = merge_lds + (size_t)(wave % half) * kMerge + lane;
+        __syncthreads();
+        if (wave >= half && wave < 2 * half) {
+            rec[0] = m;
+            rec[kWave] = l;
+#pragma unroll
+            for (int n = 0; n < NT; ++n)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) rec[(2 + n * 4 + e) * kWave] = acc[n][e];
+        }
+        __syncthreads();
+        if (wave < half) {
+            const float mo = rec[0], mn = fmaxf(m, mo);
+            const float wa = m > -__builtin_inff() ? __expf(m - mn) : 0.0f;
+            const float wb = mo > -__builtin_inff() ? __expf(mo - mn) : 0.0f;
+            l = l * wa + rec[kWave] * wb;
+            m = mn;
+#pragma unroll
+            for (int n = 0; n < NT; ++n)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) acc[n][e] = acc[n][e] * wa + rec[(2 + n * 4 + e) * kWave] * wb;
+        }
+    }
+    if (wave != 0 || col >= G) return;
+    if (row.splits <= 1) {
+        const float inv = l > 0.0f ? 1.0f / l : 0.0f;
+#pragma unroll
+        for (int h = 0; h < VH; ++h)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                typename O::T *o = out + ((size_t)b * n_heads + (size_t)g * G + col) * HD + 128 * h + DP * (4 * grp + e);
+                float r[DP];
+#pragma unroll
+                for (int j = 0; j < DP; ++j) r[j] = l > 0.0f ? acc[h * DP + j][e] * kUnscale * inv : 0.0f;
+                store_f32<O, DP>(o, r);
+            }
     } else {
         // partial record per (b, g, s, head slot): HD sums, then m, l
-        float *rec = part + ((size_t)bg * splits + s) * GM * (HD + kRecTail);
-        if (grp == 0) {
-#pragma unroll kEpiUnroll
-            for (int h = 0; h < GM; ++h) {
-                if ((uint32_t)h < G) {
+        float *rec = part + (((size_t)bg * splits + s) * rec_heads + col) * (HD + kRecTail);
 #pragma unroll
-                    for (int d = 0; d < DP; ++d) rec[h * (HD + kRecTail) + col * DP + d] = acc[h][d];
-                }
-            }
-            if (col < G) {
-                rec[col * (HD + kRecTail) + HD] = m;
-                rec[col * (HD + kRecTail) + HD + 1] = l;
-            }
+        for (int h = 0; h < VH; ++h)
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+#pragma unroll
+                for (int j = 0; j < DP; ++j) rec[128 * h + DP * (4 * grp + e) + j] = acc[h * DP + j][e] * kUnscale;
+        if (grp == 0) {
+            rec[HD] = m;
+            rec[HD + 1] = l;
         }
     }
 }
@@ -416,8 +438,10 @@ constexpr uint32_t kMaxSplits = 256;
 template <typename O, int HD, int GM>
 __global__ __launch_bounds__(kCombineThreads) void paged_decode_combine(const float *__restrict__ part,
                                                                         typename O::T *__restrict__ out,
+                                                                        const uint32_t *__restrict__ lens,
                                                                         uint32_t n_heads, uint32_t n_kv,
-                                                                        uint32_t splits) {
+                                                                        uint32_t causal, uint32_t window,
+                                                                        uint32_t alloc_splits, uint32_t bps) {
     constexpr int kParts = kCombineThreads / HD;
     constexpr int kPer = kMaxSplits / kParts;  // splits per thread at most
     constexpr int kWaves = kCombineThreads / kWave;
@@ -427,7 +451,9 @@ __global__ __launch_bounds__(kCombineThreads) void paged_decode_combine(const fl
     const uint32_t bh = blockIdx.x, h = bh % n_heads, b = bh / n_heads;
     const uint32_t G = n_heads / n_kv, g = h / G, slot = h % G;
     constexpr uint32_t kRec = GM * (HD + kRecTail);
-    const float *base = part + ((size_t)(b * n_kv + g) * splits) * kRec + slot * (HD + kRecTail);
+    const float *base = part + ((size_t)(b * n_kv + g) * alloc_splits) * kRec + slot * (HD + kRecTail);
+    const uint32_t splits = row_keys(lens[b], causal, window, bps, alloc_splits).splits;
+    if (splits <= 1) return;  // finished by its split
     const uint32_t t = threadIdx.x, d = t % HD, p = t / HD;
     float av[kPer];
 #pragma unroll
@@ -477,15 +503,19 @@ __global__ __launch_bounds__(kCombineThreads) void paged_decode_combine(const fl
 template <typename O, int HD, int GM>
 __global__ __launch_bounds__(kWave) void paged_decode_combine_wave(const float *__restrict__ part,
                                                                    typename O::T *__restrict__ out,
+                                                                   const uint32_t *__restrict__ lens,
                                                                    uint32_t n_heads, uint32_t n_kv,
-                                                                   uint32_t splits) {
+                                                                   uint32_t causal, uint32_t window,
+                                                                   uint32_t alloc_splits, uint32_t bps) {
     constexpr uint32_t kRec = HD + kRecTail;
     constexpr uint32_t LPR = HD / 4, SG = kWave / LPR;  // lanes per record, split groups
     constexpr uint32_t kPerLane = kMaxSplits / kWave;
     __shared__ float w_lds[kMaxSplits];
     const uint32_t bh = blockIdx.x, h = bh % n_heads, b = bh / n_heads;
     const uint32_t G = n_heads / n_kv, g = h / G, slot = h % G;
-    const float *base = part + ((size_t)(b * n_kv + g) * splits * GM + slot) * kRec;  // split s: + s * GM * kRec
+    const float *base = part + ((size_t)(b * n_kv + g) * alloc_splits * GM + slot) * kRec;  // split s: + s * GM * kRec
+    const uint32_t splits = row_keys(lens[b], causal, window, bps, alloc_splits).splits;
+    if (splits <= 1) return;  // finished by its split
     const uint32_t lane = threadIdx.x, dq = lane % LPR, sg = lane / LPR;
     // the first batch of record sums first: its latency overlaps the m / l
     // reductions
@@ -552,76 +582,67 @@ __global__ __launch_bounds__(kWave) void paged_decode_combine_wave(const float *
     }
 }
 
-// Split count: about kTargetWaves wavefronts when batch * n_kv is small, at
-// least kMinSplitBlocks blocks per split, at most kMaxSplits.
-// Measured (one Llama-3-8B sequence, 8 KV heads): 2048 keys took 32 us with
-// 16-block splits and 17.5 us with 2-block ones; 32768 keys did best at
-// 128 splits (1024 wavefronts) rather than 256.
-constexpr uint32_t kMinSplitBlocks = 2;
-// Build knobs: the one-wavefront combine for launches of at most
-// COMBINE_WAVE_MAX splits (1), or the 1024-thread combine always (0).
-// Measured interleaved on one box: one 2048-key sequence (64 splits) 11.96
-// against 12.16 us; one 32768-key sequence (128 splits) 35.9 against 34.0 us
-// with the wavefront form, hence the limit.
-#ifndef FELLM_ATT_COMBINE_WAVE
-#define FELLM_ATT_COMBINE_WAVE 1
-#endif
-#ifndef FELLM_ATT_COMBINE_WAVE_MAX
-#define FELLM_ATT_COMBINE_WAVE_MAX 64
-#endif
-// Build knob: wavefronts the split policy aims for.  With two blocks in
-// flight from 8-block walks, one 32768-key sequence measured 34.0-34.2 us at
-// 1024, 41.3-41.4 at 2048 and 52.3 at 512 (interleaved on one box).
-#ifndef FELLM_ATT_TARGET_WAVES
-#define FELLM_ATT_TARGET_WAVES 1024
-#endif
-constexpr uint32_t kTargetWaves = FELLM_ATT_TARGET_WAVES;
-// Build knob: blocks per wavefront from which DEPTH 2 is used.  Measured
-// (interleaved on one box): one Llama-3-8B sequence of 32768 keys (splits of
-// 16 blocks) 37.8-37.9 us from 64, 33.9 us from 4, 8 or 16; 2048 keys (splits
-// of 2 blocks) and 256 sequences x 4096 keys level.
-#ifndef FELLM_ATT_DEEP_WALK
-#define FELLM_ATT_DEEP_WALK 8
-#endif
-constexpr uint32_t kDeepWalk = FELLM_ATT_DEEP_WALK;
+// Splits of a row's keys over workgroups.
+//  * Few (row, KV head) pairs: about one workgroup per CU, at least 8 blocks
+//    each (a pair of blocks per wavefront); rows of up to 32 blocks stay whole.
+//    One row at 8 KV heads: 256 keys 6.6 us whole, 8.9 in two splits; 2048 keys
+//    9.9 us in 16 splits, 11.3 in 8; 32768 keys 27.3 in 32, 28.4 in 64.
+//  * Long rows: splits of 128 blocks (2048 keys) while the launch stays within
+//    2048 workgroups, so that a batch of mixed lengths does not wait for its
+//    longest rows.  64 rows of 256 .. 4096 keys: 123.7 us against 118.4 with
+//    splits of 64 blocks, but 64 rows of 4096 keys each 194 against 202; 256
+//    rows of 4096 keys 677 us whole, 740 in two splits.
+constexpr uint32_t kSplitTarget = 256, kMinSplitBlocks = 8, kWholeBlocks = 32;
+constexpr uint32_t kLongSplitBlocks = 128, kLongSplitMax = 2048;
 uint32_t choose_splits(uint32_t batch, uint32_t n_kv, uint32_t max_seq) {
     const uint32_t pairs = batch * n_kv;
     const uint32_t blocks = (max_seq + kBlockTokens - 1) / kBlockTokens;
-    uint32_t s = pairs >= kTargetWaves ? 1 : (kTargetWaves + pairs - 1) / pairs;
-    const uint32_t cap = blocks / kMinSplitBlocks > 0 ? blocks / kMinSplitBlocks : 1;
-    if (s > cap) s = cap;
-    if (s > kMaxSplits) s = kMaxSplits;
-    return s ? s : 1;
+    if (pairs == 0 || blocks <= kWholeBlocks) return 1;
+    uint32_t s = (kSplitTarget + pairs - 1) / pairs;
+    if (s > blocks / kMinSplitBlocks) s = blocks / kMinSplitBlocks;
+    uint32_t by_length = (blocks + kLongSplitBlocks - 1) / kLongSplitBlocks;
+    if (by_length > kLongSplitMax / pairs) by_length = kLongSplitMax / pairs;
+    if (s < by_length) s = by_length;
+    return s < kMaxSplits ? s : kMaxSplits;
 }
 
-template <typename Q, typename O, typename C, int HD, int GM>
+// Launches of at most this many workgroups request their first blocks before
+// the row length arrives (one row of 32768 keys 27.9 -> 27.3 us).
+constexpr uint32_t kEarlyGrid = 512;
+// The one-wavefront combine up to this many splits (32 splits: 27.3 us against
+// 28.5 with the 1024-thread one), the 1024-thread combine beyond.
+constexpr uint32_t kWaveCombineSplits = 64;
+
+template <typename Q, typename O, typename C, int HD>
 int launch_decode(const void *q, void *out, uint32_t batch, uint32_t n_heads, uint32_t n_kv, const uint32_t *lens,
                   uint32_t max_seq, float scale, uint32_t causal, uint32_t window, const PagedGeom &geo,
                   float *ws, uint64_t ws_bytes, hipStream_t st) {
+    const uint32_t gm = n_heads / n_kv <= 8 ? 8 : 16;
     uint32_t splits = choose_splits(batch, n_kv, max_seq);
-    const uint64_t need = (uint64_t)batch * n_kv * splits * GM * (HD + kRecTail) * 4;
+    const uint64_t need = (uint64_t)batch * n_kv * splits * gm * (HD + kRecTail) * 4;
     if (splits > 1 && (!ws || ws_bytes < need)) splits = 1;
     const uint32_t blocks = (max_seq + kBlockTokens - 1) / kBlockTokens;
-    const uint32_t bps = (blocks + splits - 1) / splits;
-    // Two blocks in flight pay off on walks of 8 blocks and more (256
-    // sequences x 4096 keys: 754 -> 720 us); splits of a few blocks do better
-    // with one.
-    if (bps >= kDeepWalk)
-        FELLM_LAUNCH((paged_decode_kernel<Q, O, C, HD, GM, 2>), dim3(batch * n_kv * splits), dim3(kWave), 0,
-                           st, static_cast<const typename Q::T *>(q), static_cast<typename O::T *>(out), ws, lens,
-                           geo.table, geo, n_heads, n_kv, scale, causal, window, splits, bps);
-    else
-        FELLM_LAUNCH((paged_decode_kernel<Q, O, C, HD, GM, 1>), dim3(batch * n_kv * splits), dim3(kWave), 0,
-                           st, static_cast<const typename Q::T *>(q), static_cast<typename O::T *>(out), ws, lens,
-                           geo.table, geo, n_heads, n_kv, scale, causal, window, splits, bps > 0 ? bps : 1);
+    const uint32_t bps = blocks ? (blocks + splits - 1) / splits : 1;
+    const uint32_t grid = batch * n_kv * splits;
+    const uint32_t lds = kDecodeWaves / 2 * (HD / 4 + 2) * kWave * sizeof(float);
+    const uint32_t early = !(causal && window) && grid <= kEarlyGrid;
+    FELLM_LAUNCH((paged_decode_kernel<Q, O, C, HD>), dim3(grid), dim3(kWave * kDecodeWaves), lds, st,
+                 static_cast<const typename Q::T *>(q), static_cast<typename O::T *>(out), ws, lens, geo, batch, n_heads,
+                 n_kv, scale, causal, window, splits, bps, gm, early);
     int rc = launch_status();
     if (rc != FELLM_OK || splits == 1) return rc;
-    if (FELLM_ATT_COMBINE_WAVE && splits <= FELLM_ATT_COMBINE_WAVE_MAX && aligned_to(ws, 16))
-        FELLM_LAUNCH((paged_decode_combine_wave<O, HD, GM>), dim3(batch * n_heads), dim3(kWave), 0, st, ws,
-                     static_cast<typename O::T *>(out), n_heads, n_kv, splits);
+    auto combine = [&]<int GM>() {
+        if (splits <= kWaveCombineSplits && aligned_to(ws, 16))
+            FELLM_LAUNCH((paged_decode_combine_wave<O, HD, GM>), dim3(batch * n_heads), dim3(kWave), 0, st, ws,
+                         static_cast<typename O::T *>(out), lens, n_heads, n_kv, causal, window, splits, bps);
+        else
+            FELLM_LAUNCH((paged_decode_combine<O, HD, GM>), dim3(batch * n_heads), dim3(kCombineThreads), 0, st, ws,
+                         static_cast<typename O::T *>(out), lens, n_heads, n_kv, causal, window, splits, bps);
+    };
+    if (gm == 8)
+        combine.template operator()<8>();
     else
-        FELLM_LAUNCH((paged_decode_combine<O, HD, GM>), dim3(batch * n_heads), dim3(kCombineThreads), 0, st, ws,
-                     static_cast<typename O::T *>(out), n_heads, n_kv, splits);
+        combine.template operator()<16>();
     return launch_status();
 }
 
@@ -629,16 +650,13 @@ template <typename Q, typename O, typename C>
 int dispatch_hd(uint32_t hd, uint32_t G, const void *q, void *out, uint32_t batch, uint32_t n_heads, uint32_t n_kv,
                 const uint32_t *lens, uint32_t max_seq, float scale, uint32_t causal, uint32_t window,
                 const PagedGeom &geo, float *ws, uint64_t ws_bytes, hipStream_t st) {
-#define FELLM_ATT(HDV, GMV)                                                                                    \
-    if (hd == HDV && G <= GMV)                                                                                 \
-        return launch_decode<Q, O, C, HDV, GMV>(q, out, batch, n_heads, n_kv, lens, max_seq, scale, causal, window, \
-                                                 geo, ws, ws_bytes, st);
-    FELLM_ATT(64, 8)
-    FELLM_ATT(64, 16)
-    FELLM_ATT(128, 8)
-    FELLM_ATT(128, 16)
-    FELLM_ATT(256, 8)
-    FELLM_ATT(256, 16)
+#define FELLM_ATT(HDV)                                                                                              \
+    if (hd == HDV)                                                                                                  \
+        return launch_decode<Q, O, C, HDV>(q, out, batch, n_heads, n_kv, lens, max_seq, scale, causal, window, geo, \
+                                           ws, ws_bytes, st);
+    FELLM_ATT(64)
+    FELLM_ATT(128)
+    FELLM_ATT(256)
 #undef FELLM_ATT
     return FELLM_ERR_SHAPE;
 }

@@ -256,11 +256,12 @@ int fellm_rocm_matvec_kquant(const void *w, uint32_t w_dtype, uint32_t rows, uin
  * head_dim 64, 128 or 256; n_heads / n_kv_heads <= 16; kv->block_size 16,
  * kv->stride = n_kv_heads * head_dim, kv_dtype F16 or BF16.
  * workspace: fellm_rocm_paged_attention_workspace() bytes for split-key
- * partial sums (used when batch * n_kv_heads is small; 16-byte aligned for
- * the fastest combine); with a null or short workspace every (row, KV head)
- * runs in one wavefront.
- * Products with the f16 cache are exact (q split into f16 high/low parts on
- * the matrix cores); accumulation, exp and the softmax run in f32.
+ * partial sums (used when batch * n_kv_heads is small or max_seq large;
+ * 16-byte aligned for the fastest combine); with a null or short workspace
+ * every (row, KV head) runs in one workgroup.
+ * Products with the cache run on the matrix cores and are exact (q and the
+ * probabilities are split into 16-bit parts); accumulation, exp and the
+ * softmax run in f32.
  */
 uint64_t fellm_rocm_paged_attention_workspace(uint32_t batch, uint32_t n_heads, uint32_t n_kv_heads,
                                               uint32_t head_dim, uint32_t max_seq);

@@ -1,0 +1,89 @@
+"""Paged decode attention at the edges of its work split: lengths around a
+block, a pair of blocks, a round of the four wavefronts' pairs and a split;
+rows that finish in one split beside rows that need several; walks long enough
+to reload the block-table lanes; windows across splits; non-finite stale bytes
+past a row's length and absent blocks.
+
+Tolerance as in test_gpu_attention.py: 2e-5 of the row's largest |V| plus an
+ulp of the output."""
+from __future__ import annotations
+
+import numpy as np
+import pytest
+
+import oracle
+from test_gpu_attention import check, make_case, run_gpu
+
+pytestmark = pytest.mark.gpu
+torch = pytest.importorskip("torch")
+
+
+@pytest.fixture(scope="module")
+def ops():
+    from fellm_amd import ops as _ops
+
+    return _ops
+
+
+def _ref(q, nh, nkv, hd, lengths, arena, table, n_logical, bb, kind, window=0):
+    return oracle.paged_attention(q, nh, nkv, hd, np.array(lengths), float(np.float32(1 / np.sqrt(hd))), arena, table,
+                                  n_logical, 1, 0, 16, bb, kind=kind, window=window)
+
+
+@pytest.mark.parametrize("kind", ["f16", "bf16"])
+@pytest.mark.parametrize("nh,nkv,hd", [(8, 2, 64), (14, 2, 128), (4, 1, 256)])
+@pytest.mark.parametrize("lengths", [[31, 32, 33, 127, 128, 129, 144, 0], [513, 1, 640, 527, 528], [4100, 40]])
+def test_lengths_around_the_split(ops, dev, lengths, nh, nkv, hd, kind):
+    rng = np.random.default_rng(sum(lengths) + hd)
+    q, arena, table, n_logical, bb, v16 = make_case(rng, lengths, nh, nkv, hd, kind)
+    got, _ = run_gpu(ops, dev, q, "f32", "f32", arena, table, n_logical, bb, lengths, nh, nkv, hd, kind)
+    check(got, _ref(q, nh, nkv, hd, lengths, arena, table, n_logical, bb, kind), v16, "f32", f"{lengths}")
+
+
+@pytest.mark.parametrize("window", [17, 600, 2048])
+def test_window_across_splits_and_table_reload(ops, dev, window):
+    """5000 keys with and without split-key scratch: one workgroup then walks
+    40 pairs per wavefront, past the 32 its table lanes hold."""
+    rng = np.random.default_rng(window)
+    nh, nkv, hd, lengths = 8, 2, 64, [5000, 700]
+    q, arena, table, n_logical, bb, v16 = make_case(rng, lengths, nh, nkv, hd, "f16")
+    for win in (window, 0):
+        ref = _ref(q, nh, nkv, hd, lengths, arena, table, n_logical, bb, "f16", window=win)
+        for workspace in ("auto", None):
+            got, _ = run_gpu(ops, dev, q, "f32", "f32", arena, table, n_logical, bb, lengths, nh, nkv, hd, "f16",
+                             window=win, workspace=workspace)
+            check(got, ref, v16, "f32", f"window {win} workspace {workspace}")
+
+
+@pytest.mark.parametrize("kind,bad", [("f16", 0x7E01), ("f16", 0x7C00), ("bf16", 0x7FC1), ("bf16", 0xFF80)])
+@pytest.mark.parametrize("length", [1, 20, 37, 600])
+def test_stale_bytes_and_absent_blocks(ops, dev, kind, bad, length):
+    """NaN or inf in every slot past the row's length changes nothing; a block
+    whose table entry is out of range contributes nothing."""
+    rng = np.random.default_rng(length)
+    nh, nkv, hd, stride = 8, 2, 128, 256
+    q, arena, table, n_logical, bb, v16 = make_case(rng, [length], nh, nkv, hd, kind)
+    ref = _ref(q, nh, nkv, hd, [length], arena, table, n_logical, bb, kind)
+    stale = arena.copy().view(np.uint16).reshape(-1, bb // 2)
+    live = np.zeros_like(stale, bool)
+    for t in range(length):
+        for v in (0, 1):
+            at = (v * 16 + t % 16) * stride
+            live[table[t // 16], at:at + stride] = True
+    stale[~live] = bad
+    got, _ = run_gpu(ops, dev, q, "f32", "f32", stale.reshape(-1).view(np.uint8), table, n_logical, bb, [length], nh, nkv,
+                     hd, kind)
+    check(got, ref, v16, "f32", "stale")
+    if length > 32:  # drop the second block: the same as attending the others
+        gone = table.copy()
+        gone[1] = 10 ** 6
+        got, _ = run_gpu(ops, dev, q, "f32", "f32", arena, gone, n_logical, bb, [length], nh, nkv, hd, kind)
+        keep = [t for t in range(length) if t // 16 != 1]
+        k16 = arena.view(np.uint16).reshape(-1, bb // 2)
+
+        def rows(v):
+            bits = np.stack([k16[table[t // 16], (v * 16 + t % 16) * stride:(v * 16 + t % 16 + 1) * stride] for t in keep])
+            return oracle.widen(np.ascontiguousarray(bits), kind).reshape(len(keep), stride)
+
+        ref = oracle.attention_f32kv(q, nh, nkv, hd, rows(0), rows(1), 0, len(keep))
+        check(got, ref, v16, "f32", "absent block")

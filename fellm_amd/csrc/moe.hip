@@ -283,6 +283,33 @@ inline DispatchGrid dispatch_grid(uint64_t n) {
     return {(uint32_t)nb, chunk};
 }
 
+// Streaming (non-temporal) or plain access to one vector.
+template <bool NT, typename V>
+__device__ __forceinline__ V load_vec(const V *p) {
+    if constexpr (NT) {
+        typedef uint32_t Words __attribute__((ext_vector_type(sizeof(V) / 4)));
+        return __builtin_bit_cast(V, __builtin_nontemporal_load(reinterpret_cast<const Words *>(p)));
+    } else {
+        return *p;
+    }
+}
+template <bool NT, typename V>
+__device__ __forceinline__ void store_vec(V *p, const V &v) {
+    if constexpr (NT) {
+        typedef uint32_t Words __attribute__((ext_vector_type(sizeof(V) / 4)));
+        __builtin_nontemporal_store(__builtin_bit_cast(Words, v), reinterpret_cast<Words *>(p));
+    } else {
+        *p = v;
+    }
+}
+
+// Bytes from which the expert rows (combine) and the grouped rows (gather) are
+// streamed: half of the 256 MB last-level cache.  Below, a caller's next or
+// previous kernel may find them there.  Measured: combine of 16384 tokens x 8
+// rows of 8 KB 261 -> 225 us in expert order and 231 -> 199 in slot order, of
+// 512 tokens 9.4 -> 10.0 (so it stays plain).
+constexpr uint64_t kStreamBytes = 128ull << 20;
+
 // grouped[i] = x[order[i] / top_k]; an invalid order entry gives a zero row.
 template <typename V>
 __global__ __launch_bounds__(256) void moe_gather_rows(const V *__restrict__ x, const uint32_t *__restrict__ order,
@@ -306,7 +333,7 @@ __global__ __launch_bounds__(256) void moe_gather_rows(const V *__restrict__ x, 
 // tail past the valid assignments) is zeroed; rows p in [t * top_k,
 // (t + 1) * top_k) are checked by token t's block.  The row is staged
 // through registers in segments of kSeg 16-byte vectors per thread.
-template <int kSeg>
+template <int kSeg, bool NT>
 __global__ __launch_bounds__(256) void moe_scatter_rows(const uint4 *__restrict__ x,
                                                         const uint32_t *__restrict__ order,
                                                         const uint32_t *__restrict__ inv, uint64_t tokens,
@@ -339,7 +366,7 @@ __global__ __launch_bounds__(256) void moe_scatter_rows(const uint4 *__restrict_
 #pragma unroll
                 for (int u = 0; u < kSeg; ++u) {
                     const uint64_t j = j0 + (uint64_t)u * 256 + t;
-                    if (j < row_vecs) dst[j] = v[u];
+                    if (j < row_vecs) store_vec<NT>(dst + j, v[u]);
                 }
             }
             for (uint32_t s = 0; s < top_k; ++s) {
@@ -359,17 +386,13 @@ __global__ __launch_bounds__(256) void moe_scatter_rows(const uint4 *__restrict_
 
 // y[t] = y0[t] (or 0) + sum over t's slots of weight * row, one token per
 // block iteration.  EXPERT_ORDER: slots in ascending (expert id, slot), rows
-// expert_out[inv[a]]; otherwise slot order, rows expert_out[a].
-template <bool EXPERT_ORDER, int VEC>
-// Build knobs: combine workgroup size and grid cap.  512 threads (one 16-byte
-// column per thread at hidden 2048) measured 3% faster than 256 in both orders.
-#ifndef FELLM_MOE_COMBINE_BLOCK
-#define FELLM_MOE_COMBINE_BLOCK 512
-#endif
-#ifndef FELLM_MOE_COMBINE_CAP
-#define FELLM_MOE_COMBINE_CAP 65536
-#endif
-__global__ __launch_bounds__(FELLM_MOE_COMBINE_BLOCK) void moe_combine_rows(const float *y0, const float *__restrict__ expert_out,
+// expert_out[inv[a]]; otherwise slot order, rows expert_out[a].  Bound by the
+// rows' bytes.  Workgroups of 1024 threads where a row has more than 512
+// vectors (top-4 rows of 16 KB 75.6 -> 67.7 us, top-8 rows of 11.5 KB 337 ->
+// 326), of 512 otherwise (top-8 rows of 8 KB 225 us, 264 with 1024, 240 with
+// 256).
+template <bool EXPERT_ORDER, int VEC, bool NT>
+__global__ __launch_bounds__(1024) void moe_combine_rows(const float *y0, const float *__restrict__ expert_out,
                                                         const uint32_t *__restrict__ ids,
                                                         const float *__restrict__ weights,
                                                         const uint32_t *__restrict__ inv, uint64_t tokens,
@@ -420,7 +443,7 @@ __global__ __launch_bounds__(FELLM_MOE_COMBINE_BLOCK) void moe_combine_rows(cons
                     const uint32_t s = s0 + u;
                     const uint32_t row = s < top_k ? srow[s] : kInvalid;
                     if (row != kInvalid)
-                        r[u] = reinterpret_cast<const Vec *>(expert_out)[(uint64_t)row * nvec + j];
+                        r[u] = load_vec<NT>(reinterpret_cast<const Vec *>(expert_out) + (uint64_t)row * nvec + j);
                 }
 #pragma unroll
                 for (int u = 0; u < 8; ++u) {
@@ -432,7 +455,7 @@ __global__ __launch_bounds__(FELLM_MOE_COMBINE_BLOCK) void moe_combine_rows(cons
                     }
                 }
             }
-            reinterpret_cast<Vec *>(y)[ybase + j] = acc;
+            store_vec<NT>(reinterpret_cast<Vec *>(y) + ybase + j, acc);
         }
         __syncthreads();
     }
@@ -562,12 +585,19 @@ extern "C" int fellm_rocm_moe_gather(const void *x, uint32_t elem_bytes, uint64_
     if (inv && vec16) {
         const uint64_t row_vecs = row_bytes / 16;
         const uint32_t grid = grid_cap(tokens, 16384);
-        if (row_vecs <= 256)
-            FELLM_LAUNCH(moe_scatter_rows<1>, dim3(grid), dim3(256), 0, st, static_cast<const uint4 *>(x), order,
-                               inv, tokens, top_k, row_vecs, static_cast<uint4 *>(grouped));
+        const bool nt = n * row_bytes >= kStreamBytes;
+#define FELLM_MOE_SCATTER(SEG, NT)                                                                                  \
+    FELLM_LAUNCH((moe_scatter_rows<SEG, NT>), dim3(grid), dim3(256), 0, st, static_cast<const uint4 *>(x), order, \
+                       inv, tokens, top_k, row_vecs, static_cast<uint4 *>(grouped))
+        if (row_vecs <= 256 && nt)
+            FELLM_MOE_SCATTER(1, true);
+        else if (row_vecs <= 256)
+            FELLM_MOE_SCATTER(1, false);
+        else if (nt)
+            FELLM_MOE_SCATTER(4, true);
         else
-            FELLM_LAUNCH(moe_scatter_rows<4>, dim3(grid), dim3(256), 0, st, static_cast<const uint4 *>(x), order,
-                               inv, tokens, top_k, row_vecs, static_cast<uint4 *>(grouped));
+            FELLM_MOE_SCATTER(4, false);
+#undef FELLM_MOE_SCATTER
         return launch_status();
     }
     const uint32_t grid = grid_cap(n, 8192);
@@ -594,22 +624,26 @@ extern "C" int fellm_rocm_moe_combine(const float *y0, const float *expert_out, 
     if (tokens == 0 || hidden == 0) return FELLM_OK;
     if (!expert_out || !weights || !y || (inv && !ids)) return FELLM_ERR_ARITY;
     hipStream_t st = as_stream(stream);
-    const uint32_t grid = grid_cap(tokens, FELLM_MOE_COMBINE_CAP);
+    const uint32_t grid = grid_cap(tokens, 65536);
     const bool vec = hidden % 4 == 0 && aligned_to(expert_out, 16) && aligned_to(y, 16) && (!y0 || aligned_to(y0, 16));
-#define FELLM_MOE_COMBINE(ORD, V)                                                                                   \
-    FELLM_LAUNCH((moe_combine_rows<ORD, V>), dim3(grid), dim3(FELLM_MOE_COMBINE_BLOCK), 0, st, y0, expert_out, ids, weights, inv, \
+    const uint32_t block = hidden / (vec ? 4 : 1) > 512 ? 1024 : 512;
+    const bool nt = n * hidden * sizeof(float) >= kStreamBytes;
+#define FELLM_MOE_COMBINE(ORD, V, NT)                                                                              \
+    FELLM_LAUNCH((moe_combine_rows<ORD, V, NT>), dim3(grid), dim3(block), 0, st, y0, expert_out, ids, weights, inv, \
                        tokens, top_k, hidden, n, y)
+#define FELLM_MOE_COMBINE_V(ORD)          \
+    if (vec && nt)                        \
+        FELLM_MOE_COMBINE(ORD, 4, true);  \
+    else if (vec)                         \
+        FELLM_MOE_COMBINE(ORD, 4, false); \
+    else                                  \
+        FELLM_MOE_COMBINE(ORD, 1, false)
     if (inv) {
-        if (vec)
-            FELLM_MOE_COMBINE(true, 4);
-        else
-            FELLM_MOE_COMBINE(true, 1);
+        FELLM_MOE_COMBINE_V(true);
     } else {
-        if (vec)
-            FELLM_MOE_COMBINE(false, 4);
-        else
-            FELLM_MOE_COMBINE(false, 1);
+        FELLM_MOE_COMBINE_V(false);
     }
+#undef FELLM_MOE_COMBINE_V
 #undef FELLM_MOE_COMBINE
     return launch_status();
 }

@@ -16,14 +16,15 @@
 // non-temporal loads; they are the only HBM traffic that scales with the
 // problem.  Each workgroup quantizes x to Q8_K in LDS (cols bytes of qs,
 // cols/16 int16 bsums, cols/256 f32 scales) while its first weight loads are
-// in flight.  A wavefront then walks units of at most 32 blocks per matrix
-// (a group of 32/cols*256 whole rows, or one 32-block pass of a long row):
-// the unit's bytes arrive by coalesced 16-byte loads (lane l, chunk 64i + l)
-// into registers one unit ahead, are written to the wavefront's LDS stage,
-// and are reduced from there by lane pairs, two lanes per block (lane half h
-// covers elements 128h .. 128h+127).  After a row's last unit, lanes
-// 0 .. 2*rows-1 fold the rows' gate and up sums in parallel and the even
-// lanes apply silu(gate) * up.
+// in flight; every wavefront then keeps the slice of x that it needs in
+// registers.  A wavefront walks units of at most 32 blocks per matrix (a group
+// of 32/cols*256 whole rows, or its share of the blocks of a longer row): the
+// unit's bytes arrive by coalesced 16-byte loads (lane l, chunk 64i + l) into
+// registers one unit ahead, are written to the wavefront's LDS stage, and are
+// reduced from there by lane pairs, two lanes per block (lane half h covers
+// elements 128h .. 128h+127).  The block values of whole rows are folded from
+// LDS in parallel lanes, one per row and matrix, and the even lanes apply
+// silu(gate) * up.
 //
 // Arithmetic.  Integer parts are exact: 4-byte dot products (v_dot4) give the
 // per-group sums, combined with the 6-bit scales/mins exactly as the CPU's
@@ -52,31 +53,17 @@
 #define FELLM_GEMV_WIDE_GRID 768
 #endif
 
-// Build knob: weight units in flight per wavefront (1 or 2 register sets).
-#ifndef FELLM_GEMV_DEPTH
-#define FELLM_GEMV_DEPTH 1
-#endif
-
 
 namespace fellm {
 namespace {
 
 constexpr int kGemvBlock = 256;
 constexpr int kGemvWaves = kGemvBlock / kWave;
-// Build knob: wavefronts per workgroup for rows of more than 32 blocks (the
-// multi-pass layout), whose workgroups each quantize all of a long x: 8
-// halves that work against 4.  Measured interleaved on one box: Llama-3-8B
-// down projection (4096 x 14336 Q4_K) 12.9 against 15.5 us; the 8B gate/up
-// shape (one pass per row) measured 16.1 against 14.4 us with 8, so it
-// keeps 4.
 // Build knob: wavefronts per workgroup for rows of at most 32 blocks.  8
 // measured slower at the 8B gate/up shape: 16.2 us with 384 workgroups, 18.8
 // with 512, against 14.5 us for 4.
 #ifndef FELLM_GEMV_ONE_WAVES
 #define FELLM_GEMV_ONE_WAVES 4
-#endif
-#ifndef FELLM_GEMV_MULTI_WAVES
-#define FELLM_GEMV_MULTI_WAVES 8
 #endif
 constexpr uint32_t kGemvMaxCols = 49152;
 // Dynamic LDS a workgroup may take: the CU's 160 KB less the kernel's static
@@ -566,17 +553,15 @@ __device__ __forceinline__ void stage_store(uint8_t *st, uint32_t lane, const St
 template <typename GW, typename UW, bool FUSED>
 constexpr uint32_t kStagePerWave = 1024 * (kChunks<GW> + (FUSED ? kChunks<UW> : 0));
 
-// GW: gate (or the only) format; UW: up format (unused unless FUSED).
-// MULTI = false (nb <= 32): a unit is a group of rp = 32/nb consecutive rows;
-//   lane pair slot s works on block s % nb of row s / nb; the lane's x slice
-//   stays in registers for the whole launch.
-// MULTI = true (nb > 32): a unit is pass p (blocks 32p ..) of one row; x
-//   slices are read from LDS per unit.
+// Rows of at most 32 blocks.  GW: gate (or the only) format; UW: up format
+// (unused unless FUSED).  A unit is a group of rp = 32/nb consecutive rows;
+// lane pair slot s works on block s % nb of row s / nb; the lane's x slice
+// stays in registers for the whole launch.
 // Each step: next unit's loads issued -> block values of the staged unit ->
 // fold buffer; after a row's last unit, lanes 0 .. mats*rows-1 each fold one
 // (row, matrix) serially over its block values from 0.0 and the even lanes
 // apply silu(gate) * up; then the next unit is written to the stage.
-template <typename GW, typename UW, bool FUSED, bool MULTI, bool PREQ, int NW = kGemvWaves>
+template <typename GW, typename UW, bool FUSED, bool PREQ, int NW = kGemvWaves>
 __global__ __launch_bounds__(NW * kWave) void kquant_gemv_kernel(const uint8_t *__restrict__ gw,
                                                                   const uint8_t *__restrict__ uw,
                                                                   const void *__restrict__ x, float *__restrict__ out,
@@ -588,7 +573,7 @@ __global__ __launch_bounds__(NW * kWave) void kquant_gemv_kernel(const uint8_t *
     const uint32_t wave = threadIdx.x / kWave, lane = threadIdx.x % kWave;
     const uint32_t h = lane & 1, slot = lane >> 1;
     const uint32_t nbp = (nb + 3) & ~3u;
-    const uint32_t fold_floats = MULTI ? kMats * nbp : kMats * rp * nbp;
+    const uint32_t fold_floats = kMats * rp * nbp;
     uint8_t *stage = reinterpret_cast<uint8_t *>(xl.fold + NW * fold_floats) + wave * kStagePerWave<GW, UW, FUSED>;
     uint8_t *ustage = stage + 1024 * kChunks<GW>;
     float *fold = xl.fold + wave * fold_floats;
@@ -596,28 +581,16 @@ __global__ __launch_bounds__(NW * kWave) void kquant_gemv_kernel(const uint8_t *
     const uint32_t g_end = rows * grb, u_end = rows * urb;
     const Rsrc wg = weight_rsrc(gw, g_end);
     const Rsrc wu = weight_rsrc(FUSED ? uw : gw, FUSED ? u_end : g_end);
-    const uint32_t passes = MULTI ? (nb + 31) / 32 : 1;
     const uint32_t wstride = gridDim.x * NW;
     const uint32_t wid = blockIdx.x * NW + wave;
 
-    // unit n of this wavefront: (first row, pass) and its byte range per matrix
-    auto unit_row = [&](uint32_t n) { return MULTI ? wid + (n / passes) * wstride : (wid + n * wstride) * rp; };
-    auto unit_pass = [&](uint32_t n) { return MULTI ? n % passes : 0u; };
-    auto range = [&](uint32_t n, uint32_t rb, uint32_t kb, uint32_t lim, uint32_t &b0, uint32_t &b1) {
-        const uint32_t r = unit_row(n), p = unit_pass(n);
-        if (r >= rows) {
-            b0 = b1 = 0;
-            return;
-        }
-        if constexpr (MULTI) {
-            b0 = r * rb + 32 * p * kb;
-            const uint32_t nblk = nb - 32 * p < 32 ? nb - 32 * p : 32;
-            b1 = b0 + nblk * kb;
-        } else {
-            b0 = r * rb;
-            b1 = b0 + rp * rb;
-            if (b1 > lim) b1 = lim;
-        }
+    // unit n of this wavefront: its first row and its byte range per matrix
+    auto unit_row = [&](uint32_t n) { return (wid + n * wstride) * rp; };
+    auto range = [&](uint32_t n, uint32_t rb, uint32_t lim, uint32_t &b0, uint32_t &b1) {
+        const uint32_t r = unit_row(n);
+        b0 = r < rows ? r * rb : 0;
+        b1 = r < rows ? b0 + rp * rb : 0;
+        if (b1 > lim) b1 = lim;
     };
 
     // Everything the prologue waits for (x, the exp table) is requested
@@ -633,114 +606,189 @@ __global__ __launch_bounds__(NW * kWave) void kquant_gemv_kernel(const uint8_t *
     Staged<GW> sg;
     Staged<UW> su;
     uint32_t gb0, gb1, ub0 = 0, ub1 = 0;
-    range(0, grb, GW::kBytes, g_end, gb0, gb1);
+    range(0, grb, g_end, gb0, gb1);
     stage_issue(wg, gb0, gb1, lane, sg);
     if constexpr (FUSED) {
-        range(0, urb, UW::kBytes, u_end, ub0, ub1);
+        range(0, urb, u_end, ub0, ub1);
         stage_issue(wu, ub0, ub1, lane, su);
     }
-#if FELLM_GEMV_DEPTH == 2
-    Staged<GW> sg2;
-    Staged<UW> su2;
-    uint32_t gb0b, gb1b, ub0b = 0, ub1b = 0;
-    range(1, grb, GW::kBytes, g_end, gb0b, gb1b);
-    stage_issue(wg, gb0b, gb1b, lane, sg2);
-    if constexpr (FUSED) {
-        range(1, urb, UW::kBytes, u_end, ub0b, ub1b);
-        stage_issue(wu, ub0b, ub1b, lane, su2);
-    }
-#endif
     if (threadIdx.x < 32) tab_lds[threadIdx.x] = tab_v;
     x_finish<PREQ>(x, nb, xl, gemv_smem, xf);
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
     __builtin_amdgcn_s_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
 
-    const uint32_t ro = MULTI ? 0 : slot / nb, bfix = MULTI ? 0 : slot - (slot / nb) * nb;
-    const bool slot_on = MULTI || ro < rp;
+    const uint32_t ro = slot / nb, b = slot - ro * nb;
+    const bool on = ro < rp;
     XHalf xh;
-    if constexpr (!MULTI) load_x(xl, bfix, h, xh);
+    load_x(xl, b, h, xh);
     stage_store(stage, lane, sg);
     if constexpr (FUSED) stage_store(ustage, lane, su);
 
     // Block values of the staged unit n (byte ranges starting at cg0 / cu0),
-    // and after a row's last unit the row folds and the stores.
+    // then the row folds and the stores.
     auto work = [&](uint32_t n, uint32_t cg0, uint32_t cu0) {
-        const uint32_t row0 = unit_row(n), p = unit_pass(n);
+        const uint32_t row0 = unit_row(n);
         wave_lds_sync();
-        const uint32_t b = MULTI ? 32 * p + slot : bfix;  // block index within its row
-        const bool on = MULTI ? b < nb : slot_on;
-        if constexpr (MULTI) load_x(xl, on ? b : 0, h, xh);
         {
-            const uint8_t *blk = stage + (cg0 & 15u) + (MULTI ? slot * GW::kBytes : ro * grb + bfix * GW::kBytes);
+            const uint8_t *blk = stage + (cg0 & 15u) + ro * grb + b * GW::kBytes;
             const float v = block_value<GW>(GW::read(blk, h), h, xh);
-            if (on && h == (GW::kBytes == 210 ? 1u : 0u)) fold[(MULTI ? 0 : ro * kMats) * nbp + b] = v;
+            if (on && h == (GW::kBytes == 210 ? 1u : 0u)) fold[ro * kMats * nbp + b] = v;
         }
         if constexpr (FUSED) {
-            const uint8_t *blk = ustage + (cu0 & 15u) + (MULTI ? slot * UW::kBytes : ro * urb + bfix * UW::kBytes);
+            const uint8_t *blk = ustage + (cu0 & 15u) + ro * urb + b * UW::kBytes;
             const float v = block_value<UW>(UW::read(blk, h), h, xh);
-            if (on && h == (UW::kBytes == 210 ? 1u : 0u)) fold[(MULTI ? 1 : ro * kMats + 1) * nbp + b] = v;
+            if (on && h == (UW::kBytes == 210 ? 1u : 0u)) fold[(ro * kMats + 1) * nbp + b] = v;
         }
         wave_lds_sync();
-        if (!MULTI || p == passes - 1) {
-            const uint32_t nf = MULTI ? kMats : kMats * rp;
-            float acc = 0.0f;
-            if (lane < nf) acc = fold_serial(fold + lane * nbp, nb, 0.0f);
-            const uint32_t nrow = MULTI ? 1 : rp;
-            if constexpr (FUSED) {
-                const float up = dpp_f32<0x101>(acc);  // row_shl:1, lane i reads lane i+1
-                const uint32_t r = row0 + lane / 2;
-                if (lane < 2 * nrow && (lane & 1) == 0 && r < rows) out[r] = silu(acc, tab_lds) * up;
-            } else {
-                if (lane < nrow && row0 + lane < rows) out[row0 + lane] = acc;
-            }
-            wave_lds_sync();
+        float acc = 0.0f;
+        if (lane < kMats * rp) acc = fold_serial(fold + lane * nbp, nb, 0.0f);
+        if constexpr (FUSED) {
+            const float up = dpp_f32<0x101>(acc);  // row_shl:1, lane i reads lane i+1
+            const uint32_t r = row0 + lane / 2;
+            if (lane < 2 * rp && (lane & 1) == 0 && r < rows) out[r] = silu(acc, tab_lds) * up;
+        } else {
+            if (lane < rp && row0 + lane < rows) out[row0 + lane] = acc;
         }
+        wave_lds_sync();
     };
 
-#if FELLM_GEMV_DEPTH == 2
-    // Two units in flight: register sets A (sg, su) and B (sg2, su2) take
-    // alternate units; the LDS stage holds the unit being reduced.
-    for (uint32_t n = 0;; n += 2) {
-        if (unit_row(n) >= rows) break;
-        uint32_t cg0 = gb0, cu0 = ub0;
-        range(n + 2, grb, GW::kBytes, g_end, gb0, gb1);
-        stage_issue(wg, gb0, gb1, lane, sg);
-        if constexpr (FUSED) {
-            range(n + 2, urb, UW::kBytes, u_end, ub0, ub1);
-            stage_issue(wu, ub0, ub1, lane, su);
-        }
-        work(n, cg0, cu0);
-        stage_store(stage, lane, sg2);
-        if constexpr (FUSED) stage_store(ustage, lane, su2);
-        if (unit_row(n + 1) >= rows) break;
-        cg0 = gb0b;
-        cu0 = ub0b;
-        range(n + 3, grb, GW::kBytes, g_end, gb0b, gb1b);
-        stage_issue(wg, gb0b, gb1b, lane, sg2);
-        if constexpr (FUSED) {
-            range(n + 3, urb, UW::kBytes, u_end, ub0b, ub1b);
-            stage_issue(wu, ub0b, ub1b, lane, su2);
-        }
-        work(n + 1, cg0, cu0);
-        stage_store(stage, lane, sg);
-        if constexpr (FUSED) stage_store(ustage, lane, su);
-    }
-#else
     for (uint32_t n = 0;; ++n) {
         if (unit_row(n) >= rows) break;
         const uint32_t cg0 = gb0, cu0 = ub0;  // staged unit's byte ranges start here
-        range(n + 1, grb, GW::kBytes, g_end, gb0, gb1);
+        range(n + 1, grb, g_end, gb0, gb1);
         stage_issue(wg, gb0, gb1, lane, sg);
         if constexpr (FUSED) {
-            range(n + 1, urb, UW::kBytes, u_end, ub0, ub1);
+            range(n + 1, urb, u_end, ub0, ub1);
             stage_issue(wu, ub0, ub1, lane, su);
         }
         work(n, cg0, cu0);
         stage_store(stage, lane, sg);
         if constexpr (FUSED) stage_store(ustage, lane, su);
     }
-#endif
+}
+
+// Rows of more than 32 blocks.  A row's blocks are divided over `passes`
+// wavefronts (at most 32 each), so that a wavefront's x slice stays in
+// registers for the launch; a workgroup of passes * groups wavefronts works on
+// `groups` rows at a time.  (One wavefront walking a row's passes re-read its
+// x slice from LDS for every 32 blocks, at an eight-way bank conflict, and
+// folded its row in a single lane: 8192 x 28672 Q4_K 41.2 -> 28.4 us, Q6_K 58.6
+// -> 43.3, 4096 x 14336 Q4_K 13.0 -> 11.3, 5120 x 13824 20.0 -> 13.2; with 8
+// wavefronts per workgroup instead of 16 31.1, 46.0, 11.5 and 13.5.)  The block values of kFoldRows rows per
+// group collect in LDS; after a barrier one wavefront, another for every
+// batch, folds all of them, a lane per (row, matrix), while the others go on
+// into the second fold buffer.
+constexpr uint32_t kFoldRows = 4;
+constexpr uint32_t gemv_pass_lds(uint32_t nb, uint32_t passes, uint32_t groups, uint32_t mats, uint32_t stage) {
+    const uint32_t nbp = (nb + 3) & ~3u;
+    return gemv_fold_off(nb) + 2 * groups * kFoldRows * mats * nbp * 4 + passes * groups * stage;
+}
+
+template <typename GW, typename UW, bool FUSED, bool PREQ, int MAXW>
+__global__ __launch_bounds__(MAXW * kWave) void kquant_gemv_passes(const uint8_t *__restrict__ gw,
+                                                                    const uint8_t *__restrict__ uw,
+                                                                    const void *__restrict__ x, float *__restrict__ out,
+                                                                    uint32_t rows, uint32_t nb, uint32_t passes,
+                                                                    uint32_t groups) {
+    constexpr uint32_t kMats = FUSED ? 2 : 1;
+    extern __shared__ __align__(16) uint8_t gemv_smem[];
+    __shared__ uint64_t tab_lds[32];
+    const XLds xl = carve_lds(gemv_smem, nb);
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave), lane = threadIdx.x % kWave;
+    const uint32_t h = lane & 1, slot = lane >> 1;
+    const uint32_t nbp = (nb + 3) & ~3u;
+    const uint32_t pass = wave % passes, group = wave / passes, waves = passes * groups;
+    const uint32_t per = (nb + passes - 1) / passes, first = pass * per;
+    const uint32_t mine = first < nb ? (nb - first < per ? nb - first : per) : 0;
+    const uint32_t batch_floats = groups * kFoldRows * kMats * nbp;
+    uint8_t *stage = reinterpret_cast<uint8_t *>(xl.fold + 2 * batch_floats) + wave * kStagePerWave<GW, UW, FUSED>;
+    uint8_t *ustage = stage + 1024 * kChunks<GW>;
+    const uint32_t grb = nb * GW::kBytes, urb = nb * UW::kBytes;
+    const Rsrc wg = weight_rsrc(gw, rows * grb);
+    const Rsrc wu = weight_rsrc(FUSED ? uw : gw, FUSED ? rows * urb : rows * grb);
+
+    auto row_of = [&](uint32_t n, uint32_t g) { return (n * gridDim.x + blockIdx.x) * groups + g; };
+    const uint32_t steps = (rows + gridDim.x * groups - 1) / (gridDim.x * groups);
+    auto range = [&](uint32_t n, uint32_t rb, uint32_t kb, uint32_t &b0, uint32_t &b1) {
+        const uint32_t r = row_of(n, group);
+        b0 = r < rows ? r * rb + first * kb : 0;
+        b1 = r < rows ? b0 + mine * kb : 0;
+    };
+
+    // x and the exp table before the first unit's weights, as in the kernel above.
+    XFirst<PREQ> xf;
+    x_issue<PREQ>(x, nb, xf);
+    uint64_t tab_v = 0;
+    {
+        constexpr ExpfTable T = make_expf_table();
+        if (threadIdx.x < 32) tab_v = T.tab[threadIdx.x];
+    }
+    Staged<GW> sg;
+    Staged<UW> su;
+    uint32_t gb0, gb1, ub0 = 0, ub1 = 0;
+    auto issue = [&](uint32_t n) {
+        range(n, grb, GW::kBytes, gb0, gb1);
+        stage_issue(wg, gb0, gb1, lane, sg);
+        if constexpr (FUSED) {
+            range(n, urb, UW::kBytes, ub0, ub1);
+            stage_issue(wu, ub0, ub1, lane, su);
+        }
+    };
+    auto store = [&] {
+        stage_store(stage, lane, sg);
+        if constexpr (FUSED) stage_store(ustage, lane, su);
+    };
+    auto barrier = [&] {  // orders LDS only: the weight loads stay in flight
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+        __builtin_amdgcn_s_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+    };
+    issue(0);
+    if (threadIdx.x < 32) tab_lds[threadIdx.x] = tab_v;
+    x_finish<PREQ>(x, nb, xl, gemv_smem, xf);
+    barrier();
+    const bool on = slot < mine;
+    XHalf xh;
+    load_x(xl, on ? first + slot : 0, h, xh);
+    store();
+
+    uint32_t turn = 0;
+    for (uint32_t n0 = 0; n0 < steps; n0 += kFoldRows) {
+        float *fold = xl.fold + (n0 / kFoldRows % 2) * batch_floats;
+        const uint32_t n1 = steps - n0 < kFoldRows ? steps - n0 : kFoldRows;
+        for (uint32_t i = 0; i < n1; ++i) {
+            const uint32_t cg0 = gb0, cu0 = ub0;  // the staged unit starts here
+            issue(n0 + i + 1);
+            wave_lds_sync();
+            float *f = fold + (group * kFoldRows + i) * kMats * nbp + first + slot;
+            {
+                const float v = block_value<GW>(GW::read(stage + (cg0 & 15u) + slot * GW::kBytes, h), h, xh);
+                if (on && h == (GW::kBytes == 210 ? 1u : 0u)) f[0] = v;
+            }
+            if constexpr (FUSED) {
+                const float v = block_value<UW>(UW::read(ustage + (cu0 & 15u) + slot * UW::kBytes, h), h, xh);
+                if (on && h == (UW::kBytes == 210 ? 1u : 0u)) f[nbp] = v;
+            }
+            wave_lds_sync();
+            store();
+        }
+        barrier();
+        if (wave == turn) {
+            const uint32_t e = lane / kMats, g = e / kFoldRows, i = e % kFoldRows;
+            const uint32_t r = row_of(n0 + i, g);
+            const bool live = g < groups && i < n1 && r < rows;
+            float acc = 0.0f;
+            if (live) acc = fold_serial(fold + lane * nbp, nb, 0.0f);
+            if constexpr (FUSED) {
+                const float up = dpp_f32<0x101>(acc);  // row_shl:1, lane i reads lane i+1
+                if (live && (lane & 1) == 0) out[r] = silu(acc, tab_lds) * up;
+            } else {
+                if (live) out[r] = acc;
+            }
+        }
+        turn = turn + 1 < waves ? turn + 1 : 0;
+    }
 }
 
 // Rows whose bytes do not end on a 16-byte boundary (Q6_K rows of nb % 8 != 0
@@ -850,23 +898,35 @@ int launch_gemv(const void *gw, const void *uw, const void *x, float *out, uint3
             constexpr int NWO = FELLM_GEMV_ONE_WAVES;
             const uint32_t lds = gemv_lds_bytes(nb, mats * rp * nbp, NWO) + NWO * kStagePerWave<GW, UW, FUSED>;
             const uint32_t units = (n + rp - 1) / rp;
-            const uint32_t grid = gemv_grid<PREQ>(kquant_gemv_kernel<GW, UW, FUSED, false, PREQ, NWO>, lds, units, NWO);
-            FELLM_LAUNCH((kquant_gemv_kernel<GW, UW, FUSED, false, PREQ, NWO>), dim3(grid), dim3(NWO * kWave), lds, s, g, u, x,
+            const uint32_t grid = gemv_grid<PREQ>(kquant_gemv_kernel<GW, UW, FUSED, PREQ, NWO>, lds, units, NWO);
+            FELLM_LAUNCH((kquant_gemv_kernel<GW, UW, FUSED, PREQ, NWO>), dim3(grid), dim3(NWO * kWave), lds, s, g, u, x,
                                out + r0, n, nb, rp);
         } else {
-            auto go_multi = [&]<int NW>() {
-                const uint32_t lds = gemv_lds_bytes(nb, mats * nbp, NW) + NW * kStagePerWave<GW, UW, FUSED>;
-                const uint32_t grid = gemv_grid<PREQ>(kquant_gemv_kernel<GW, UW, FUSED, true, PREQ, NW>, lds, n, NW);
-                FELLM_LAUNCH((kquant_gemv_kernel<GW, UW, FUSED, true, PREQ, NW>), dim3(grid), dim3(NW * kWave), lds, s, g,
-                             u, x, out + r0, n, nb, 1u);
+            // As many groups as fit MAXW wavefronts and the LDS (half of them
+            // where all rows are one step of that grid, so that two
+            // workgroups' prologues share a CU: 2048 x 8448 Q4_K 8.2 -> 7.4
+            // us); among those of at least half as many, the one that leaves
+            // the fewest group slots of the last step empty.
+            constexpr int MAXW = FUSED ? 8 : 16;
+            const uint32_t passes = (nb + 31) / 32;
+            auto lds_of = [&](uint32_t g) { return gemv_pass_lds(nb, passes, g, mats, kStagePerWave<GW, UW, FUSED>); };
+            uint32_t most = MAXW / passes;
+            while (most > 1 && lds_of(most) > kGemvLdsLimit) --most;
+            if (n <= most * (uint32_t)cu_count()) most = (most + 1) / 2;
+            auto grid_of = [&](uint32_t g) {
+                uint32_t per_cu = kGemvLdsLimit / lds_of(g);
+                if (per_cu > (uint32_t)MAXW / (passes * g)) per_cu = MAXW / (passes * g);
+                const uint32_t all = (uint32_t)cu_count() * (per_cu ? per_cu : 1), need = (n + g - 1) / g;
+                return need < all ? need : all;
             };
-            // FELLM_GEMV_MULTI_WAVES wavefronts while their stages and x fit the
-            // workgroup's LDS (fused Q5_K / Q6_K rows of ~40k columns do not).
-            constexpr int NWM = FELLM_GEMV_MULTI_WAVES;
-            if (gemv_lds_bytes(nb, mats * nbp, NWM) + NWM * kStagePerWave<GW, UW, FUSED> <= kGemvLdsLimit)
-                go_multi.template operator()<NWM>();
-            else
-                go_multi.template operator()<kGemvWaves>();
+            uint32_t groups = most;
+            uint64_t best = ~0ull;
+            for (uint32_t g = most; 2 * g >= most && g > 0; --g) {
+                const uint64_t per_step = (uint64_t)grid_of(g) * g, slots = (n + per_step - 1) / per_step * per_step;
+                if (slots < best) best = slots, groups = g;
+            }
+            FELLM_LAUNCH((kquant_gemv_passes<GW, UW, FUSED, PREQ, MAXW>), dim3(grid_of(groups)),
+                         dim3(passes * groups * kWave), lds_of(groups), s, g, u, x, out + r0, n, nb, passes, groups);
         }
         const int rc = launch_status();
         if (rc != FELLM_OK) return rc;

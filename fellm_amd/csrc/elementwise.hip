@@ -158,10 +158,15 @@ __global__ __launch_bounds__(kEwBlock) void silu_fast_bound_kernel(uint32_t *__r
     if (threadIdx.x % kWave == 0) atomicMax(max_dist, m);
 }
 
-// VEC = 8 elements: 16 B for 16-bit types, 32 B for f32.
+// VEC: 16 bytes of the 16-bit types, and of f32 to f32: with 8 f32 elements
+// (32 bytes a lane, so an instruction covers every other 16 bytes) SwiGLU of
+// 4096 x 14336 f32 measured 131.7 against 110.4 us, the add 136.3 against 122.8.
+template <typename I, typename O>
+constexpr int kEwVec = sizeof(typename I::T) + sizeof(typename O::T) == 8 ? 4 : 8;
+
 template <typename I, typename O>
 int launch_silu(const void *g, const void *u, void *out, uint64_t n, hipStream_t s) {
-    constexpr int VEC = 8, UNROLL = FELLM_SWIGLU_UNROLL;
+    constexpr int VEC = kEwVec<I, O>, UNROLL = FELLM_SWIGLU_UNROLL;
     using TI = typename I::T;
     using TO = typename O::T;
     if (!aligned_to(g, sizeof(TI) * VEC) || !aligned_to(u, sizeof(TI) * VEC) ||
@@ -182,7 +187,7 @@ int launch_silu(const void *g, const void *u, void *out, uint64_t n, hipStream_t
 
 template <typename I, typename O>
 int launch_add(const void *a, const void *b, void *out, uint64_t n, hipStream_t s) {
-    constexpr int VEC = 8;
+    constexpr int VEC = kEwVec<I, O>;
     using TI = typename I::T;
     using TO = typename O::T;
     if (!aligned_to(a, sizeof(TI) * VEC) || !aligned_to(b, sizeof(TI) * VEC) ||

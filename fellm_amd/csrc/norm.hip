@@ -312,14 +312,18 @@ int launch_fast(const void *x, const void *r, void *h, const float *w, void *y, 
 template <typename A, typename O>
 int launch_typed(const void *x, const void *r, void *h, const float *w, void *y, uint32_t group,
                  uint64_t rows, float eps, hipStream_t s) {
-    constexpr int VEC = 8;
+    // Chunks of one 16-byte access: f32 rows to f32 in chunks of 8 (32 bytes a
+    // lane, so an instruction covers every other 16 bytes) measured 52.0
+    // against 44.6 us at 4096 x 4096 with a residual, 27.0 against 23.7
+    // without, 5.0 against 4.65 us for one row.  M chunks for each 8 elements.
+    constexpr int VEC = sizeof(typename A::T) + sizeof(typename O::T) == 8 ? 4 : 8, M = 8 / VEC;
     const bool vec_ok = group % VEC == 0 && aligned_to(x, 16) && aligned_to(y, 16) &&
-                        aligned_to(w, 32) && (!r || aligned_to(r, 16)) && (!h || aligned_to(h, 16));
+                        aligned_to(w, sizeof(float) * VEC) && (!r || aligned_to(r, 16)) && (!h || aligned_to(h, 16));
     if (vec_ok) {
         // Few rows (decode): wide blocks keep more bytes in flight per CU.
-        if (rows < 1024 && group <= 1024 * VEC * 2) {
-            if (group <= 1024 * VEC) return launch_fast<A, O, 1024, VEC, 1>(x, r, h, w, y, group, rows, eps, s);
-            return launch_fast<A, O, 1024, VEC, 2>(x, r, h, w, y, group, rows, eps, s);
+        if (rows < 1024 && group <= 1024 * 8 * 2) {
+            if (group <= 1024 * 8) return launch_fast<A, O, 1024, VEC, M>(x, r, h, w, y, group, rows, eps, s);
+            return launch_fast<A, O, 1024, VEC, 2 * M>(x, r, h, w, y, group, rows, eps, s);
         }
         // Many rows of at most 8 KB: one wavefront per row.
         constexpr uint32_t WV = 16 / sizeof(typename A::T);  // elements per 16-byte chunk
@@ -330,20 +334,20 @@ int launch_typed(const void *x, const void *r, void *h, const float *w, void *y,
             if (nch <= 4) return launch_wave<A, O, 4>(x, r, h, w, y, group, rows, eps, s);
             return launch_wave<A, O, 8>(x, r, h, w, y, group, rows, eps, s);
         }
-        if (FELLM_NORM_PIPE && r && h && group > 256 * VEC && group <= 512 * VEC) {
+        if (FELLM_NORM_PIPE && r && h && group > 256 * 8 && group <= 512 * 8) {
             using TA = typename A::T;
             using TO = typename O::T;
             const uint32_t grid = (uint32_t)std::min<uint64_t>(rows, (uint64_t)cu_count() * FELLM_NORM_PIPE);
-            FELLM_LAUNCH((add_rmsnorm_pipe_kernel<A, O, 512, VEC, 1>), dim3(grid), dim3(512), 0, s, (const TA *)x,
+            FELLM_LAUNCH((add_rmsnorm_pipe_kernel<A, O, 512, VEC, M>), dim3(grid), dim3(512), 0, s, (const TA *)x,
                          (const TA *)r, (TA *)h, w, (TO *)y, group, (uint32_t)rows, eps);
             return launch_status();
         }
-        if (FELLM_NORM_PREFILL_BLOCK == 512 && group > 256 * VEC && group <= 512 * VEC)
-            return launch_fast<A, O, 512, VEC, 1>(x, r, h, w, y, group, rows, eps, s);
-        if (group <= 256 * VEC) return launch_fast<A, O, 256, VEC, 1>(x, r, h, w, y, group, rows, eps, s);
-        if (group <= 256 * VEC * 2) return launch_fast<A, O, 256, VEC, 2>(x, r, h, w, y, group, rows, eps, s);
-        if (group <= 256 * VEC * 4) return launch_fast<A, O, 256, VEC, 4>(x, r, h, w, y, group, rows, eps, s);
-        if (group <= 256 * VEC * 8) return launch_fast<A, O, 256, VEC, 8>(x, r, h, w, y, group, rows, eps, s);
+        if (FELLM_NORM_PREFILL_BLOCK == 512 && group > 256 * 8 && group <= 512 * 8)
+            return launch_fast<A, O, 512, VEC, M>(x, r, h, w, y, group, rows, eps, s);
+        if (group <= 256 * 8) return launch_fast<A, O, 256, VEC, M>(x, r, h, w, y, group, rows, eps, s);
+        if (group <= 256 * 8 * 2) return launch_fast<A, O, 256, VEC, 2 * M>(x, r, h, w, y, group, rows, eps, s);
+        if (group <= 256 * 8 * 4) return launch_fast<A, O, 256, VEC, 4 * M>(x, r, h, w, y, group, rows, eps, s);
+        if (group <= 256 * 8 * 8) return launch_fast<A, O, 256, VEC, 8 * M>(x, r, h, w, y, group, rows, eps, s);
     }
     using TA = typename A::T;
     using TO = typename O::T;

@@ -145,7 +145,15 @@ def lib() -> C.CDLL:
     return _lib
 
 
+# Bound functions by name: the attribute lookup on the loaded library costs
+# about as much as the call itself.
+_fns: dict[str, C._CFuncPtr] = {}
+
+
 def call(name: str, *args) -> None:
-    rc = getattr(lib(), name)(*args)
+    fn = _fns.get(name)
+    if fn is None:
+        fn = _fns[name] = getattr(lib(), name)
+    rc = fn(*args)
     if rc != 0:
         raise FellmRocmError(name, rc)

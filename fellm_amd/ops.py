@@ -20,12 +20,13 @@ from .abi import DType
 
 _ACT = {torch.float32: DType.F32, torch.float16: DType.F16, torch.bfloat16: DType.BF16}
 _TORCH = {v: k for k, v in _ACT.items()}
+_ACT_CODE = {k: int(v) for k, v in _ACT.items()}
 QTYPES = {"q4k": (DType.Q4K, 144), "q5k": (DType.Q5K, 176), "q6k": (DType.Q6K, 210)}
 
 
 def _code(t: torch.Tensor) -> int:
     try:
-        return int(_ACT[t.dtype])
+        return _ACT_CODE[t.dtype]
     except KeyError as e:
         raise TypeError(f"unsupported activation dtype {t.dtype}") from e
 
@@ -34,7 +35,7 @@ def _dev(*ts: torch.Tensor | None) -> None:
     for t in ts:
         if t is None:
             continue
-        if t.device.type != "cuda":
+        if not t.is_cuda:
             raise ValueError("fellm_amd ops need device tensors (no CPU fallback)")
         if not t.is_contiguous():
             raise ValueError("fellm_amd ops need contiguous tensors")
@@ -44,8 +45,16 @@ def _p(t: torch.Tensor | None) -> int | None:
     return None if t is None else t.data_ptr()
 
 
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+
+
 def _stream() -> int:
-    return torch.cuda.current_stream().cuda_stream
+    """The handle of torch's current stream on the current device.  Read
+    without building a Stream object where torch offers that: 0.3 against 2.6
+    us, of the 7 to 8 us a call of a small op takes on the host."""
+    if _raw_stream is None:
+        return torch.cuda.current_stream().cuda_stream
+    return _raw_stream(torch.cuda.current_device())
 
 
 def add_rmsnorm(x, residual, weight, eps: float, *, h_out=None, y_out=None, y_dtype=None, store_h=True):

@@ -100,6 +100,7 @@ struct CacheF16 {
         y = y - (float)h[1];
         return __builtin_bit_cast(uint32_t, h);
     }
+    __device__ static float widen(uint32_t low16) { return (float)__builtin_bit_cast(_Float16, (uint16_t)low16); }
     __device__ static f32x4 mfma(u32x4 a, u32x4 b, f32x4 c) {
         return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(half8_t, a), __builtin_bit_cast(half8_t, b), c, 0,
                                                       0, 0);
@@ -119,6 +120,7 @@ struct CacheBF16 {
         y = y - __uint_as_float(u & 0xffff0000u);
         return u;
     }
+    __device__ static float widen(uint32_t low16) { return __uint_as_float(low16 << 16); }
     __device__ static f32x4 mfma(u32x4 a, u32x4 b, f32x4 c) {
         return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf8_t, a), __builtin_bit_cast(bf8_t, b), c, 0, 0,
                                                        0);
@@ -168,7 +170,7 @@ __device__ __forceinline__ float rows_max(float v) {
 // dim (64, 128 or 256).  rec_heads: head slots of a partial record.  early:
 // the first blocks are requested before the row length is known.
 template <typename Q, typename O, typename C, int HD>
-__global__ __launch_bounds__(kWave * kDecodeWaves) void paged_decode_kernel(const typename Q::T *__restrict__ q,
+__global__ __launch_bounds__(kWave * kDecodeWaves, HD == 64 && C::kParts == 2 ? 4 : 1) void paged_decode_kernel(const typename Q::T *__restrict__ q,
                                                              typename O::T *__restrict__ out,
                                                              float *__restrict__ part, const uint32_t *__restrict__ lens,
                                                              PagedGeom geo, uint32_t batch, uint32_t n_heads,
@@ -191,11 +193,11 @@ __global__ __launch_bounds__(kWave * kDecodeWaves) void paged_decode_kernel(cons
     const uint32_t row_bytes = geo.stride * 2;
     const size_t table_base = ((size_t)b * geo.n_layers + geo.layer) * geo.n_logical;
 
-    // This wavefront's pairs of blocks: first + 2 (wave + kDecodeWaves n), n =
-    // 0, 1, ..  Lane l holds the physical block (~0: none, or at or past lim)
-    // of block l % 2 of pair tab0 + l / 2; a walk of more than 32 pairs reloads.
-    uint32_t tab = ~0u, tab0 = 0;
-    auto pair_block = [&](uint32_t first, uint32_t n) { return first + 2 * (wave + kDecodeWaves * n); };
+    // This wavefront's pairs of blocks: first + 2 (way + ways n), n = 0, 1, ..
+    // Lane l holds the physical block (~0: none, or at or past lim) of block
+    // l % 2 of pair tab0 + l / 2; a walk of more than 32 pairs reloads.
+    uint32_t tab = ~0u, tab0 = 0, way = wave, ways = kDecodeWaves;
+    auto pair_block = [&](uint32_t first, uint32_t n) { return first + 2 * (way + ways * n); };
     auto load_table = [&](uint32_t first, uint32_t n, uint32_t lim) {
         tab0 = n;
         const uint32_t blk = pair_block(first, n + lane / 2) + lane % 2;
@@ -290,47 +292,50 @@ __global__ __launch_bounds__(kWave * kDecodeWaves) void paged_decode_kernel(cons
     }
 
     f32x4 acc[NT];  // tile (h, j) of lane (col, grp): dims 128h + DP (4 grp + e) + j of head slot col
+    float m, l;     // running max, this lane's part of the denominator
+    auto clear = [&] {
+        m = -__builtin_inff();
+        l = 0.0f;
 #pragma unroll
-    for (int n = 0; n < NT; ++n) acc[n] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-    float m = -__builtin_inff(), l = 0.0f;  // running max, this lane's part of the denominator
-
-    for (uint32_t n = 0; pair_block(blk0, n) < blk1; ++n) {
-        // S^T[token 4 grp + e][head slot col] of both blocks
+        for (int n = 0; n < NT; ++n) acc[n] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+    };
+    // p[i]: score of token 4 grp + i % 4 of block i / 4 of pair n with head slot col
+    auto scores = [&](float (&p)[8]) {
         f32x4 sc[2], sl[2];
 #pragma unroll
         for (int u = 0; u < 2; ++u) sc[u] = sl[u] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
         for (int c = 0; c < NC; ++c)
 #pragma unroll
-            for (int p = 0; p < C::kParts; ++p)
+            for (int x = 0; x < C::kParts; ++x)
 #pragma unroll
                 for (int u = 0; u < 2; ++u) {
                     // the parts below the first in a sum of their own
-                    f32x4 &d = p ? sl[u] : sc[u];
-                    d = C::mfma(kr[u][c], qb[c][p], d);
+                    f32x4 &d = x ? sl[u] : sc[u];
+                    d = C::mfma(kr[u][c], qb[c][x], d);
                 }
-        if (n + 1 - tab0 == (uint32_t)kWave / 2) load_table(blk0, n + 1, blk1);
-        const Pair next = pair_at(n + 1);
-        __builtin_amdgcn_sched_barrier(0);  // a second register set of K would cost occupancy
-        load_k(next);
-
-        const uint32_t t0 = pair_block(blk0, n) * kBlockTokens;
-        const bool edge = t0 < row.lo || t0 + 2 * kBlockTokens > row.seq || !cur.ok[0] || !cur.ok[1];
-        float p[8], mx = -__builtin_inff();
 #pragma unroll
         for (int i = 0; i < 8; ++i) p[i] = (sc[i / 4][i % 4] + sl[i / 4][i % 4]) * scale;
-        if (edge) {
+    };
+    // Tokens outside the row's keys: -inf scores, zero V.
+    auto mask = [&](uint32_t n, float (&p)[8]) {
+        const uint32_t t0 = pair_block(blk0, n) * kBlockTokens;
+        const bool edge = t0 < row.lo || t0 + 2 * kBlockTokens > row.seq || !cur.ok[0] || !cur.ok[1];
+        if (!edge) return;
 #pragma unroll
-            for (int i = 0; i < 8; ++i) {
-                const uint32_t t = t0 + (i / 4) * kBlockTokens + 4 * grp + i % 4;
-                const bool on = cur.ok[i / 4] && t >= row.lo && t < row.seq;
-                if (!on) p[i] = -__builtin_inff();
+        for (int i = 0; i < 8; ++i) {
+            const uint32_t t = t0 + (i / 4) * kBlockTokens + 4 * grp + i % 4;
+            const bool on = cur.ok[i / 4] && t >= row.lo && t < row.seq;
+            if (!on) p[i] = -__builtin_inff();
 #pragma unroll
-                for (int h = 0; h < VH; ++h)
+            for (int h = 0; h < VH; ++h)
 #pragma unroll
-                    for (int w = 0; w < DP / 2; ++w) vr[i][h][w] = on ? vr[i][h][w] : 0u;
-            }
+                for (int w = 0; w < DP / 2; ++w) vr[i][h][w] = on ? vr[i][h][w] : 0u;
         }
+    };
+    // Scores to probabilities times kPScale against the running maximum.
+    auto soften = [&](float (&p)[8]) {
+        float mx = -__builtin_inff();
 #pragma unroll
         for (int i = 0; i < 8; ++i) mx = fmaxf(mx, p[i]);
         const float mn = fmaxf(m, rows_max(mx));
@@ -347,6 +352,18 @@ __global__ __launch_bounds__(kWave * kDecodeWaves) void paged_decode_kernel(cons
             l += p[i];
             p[i] *= C::kPScale;
         }
+    };
+
+    clear();
+    for (uint32_t n = 0; pair_block(blk0, n) < blk1; ++n) {
+        float p[8];
+        scores(p);
+        if (n + 1 - tab0 == (uint32_t)kWave / 2) load_table(blk0, n + 1, blk1);
+        const Pair next = pair_at(n + 1);
+        __builtin_amdgcn_sched_barrier(0);  // a second register set of K would cost occupancy
+        load_k(next);
+        mask(n, p);
+        soften(p);
         u32x4 pb[C::kParts];
         split8<C>(p, pb);
 #pragma unroll
@@ -398,32 +415,75 @@ __global__ __launch_bounds__(kWave * kDecodeWaves) void paged_decode_kernel(cons
                 for (int e = 0; e < 4; ++e) acc[n][e] = acc[n][e] * wa + rec[(2 + n * 4 + e) * kWave] * wb;
         }
     }
-    if (wave != 0 || col >= G) return;
-    if (row.splits <= 1) {
-        const float inv = l > 0.0f ? 1.0f / l : 0.0f;
+    if (wave != 0) return;
+    auto store = [&] {
+        if (col >= G) return;
+        if (row.splits <= 1) {
+            const float inv = l > 0.0f ? 1.0f / l : 0.0f;
 #pragma unroll
-        for (int h = 0; h < VH; ++h)
+            for (int h = 0; h < VH; ++h)
 #pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                typename O::T *o = out + ((size_t)b * n_heads + (size_t)g * G + col) * HD + 128 * h + DP * (4 * grp + e);
-                float r[DP];
+                for (int e = 0; e < 4; ++e) {
+                    typename O::T *o =
+                        out + ((size_t)b * n_heads + (size_t)g * G + col) * HD + 128 * h + DP * (4 * grp + e);
+                    float r[DP];
 #pragma unroll
-                for (int j = 0; j < DP; ++j) r[j] = l > 0.0f ? acc[h * DP + j][e] * kUnscale * inv : 0.0f;
-                store_f32<O, DP>(o, r);
+                    for (int j = 0; j < DP; ++j) r[j] = l > 0.0f ? acc[h * DP + j][e] * kUnscale * inv : 0.0f;
+                    store_f32<O, DP>(o, r);
+                }
+        } else {
+            // partial record per (b, g, s, head slot): HD sums, then m, l
+            float *rec = part + (((size_t)bg * splits + s) * rec_heads + col) * (HD + kRecTail);
+#pragma unroll
+            for (int h = 0; h < VH; ++h)
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+#pragma unroll
+                    for (int j = 0; j < DP; ++j) rec[128 * h + DP * (4 * grp + e) + j] = acc[h * DP + j][e] * kUnscale;
+            if (grp == 0) {
+                rec[HD] = m;
+                rec[HD + 1] = l;
             }
-    } else {
-        // partial record per (b, g, s, head slot): HD sums, then m, l
-        float *rec = part + (((size_t)bg * splits + s) * rec_heads + col) * (HD + kRecTail);
-#pragma unroll
-        for (int h = 0; h < VH; ++h)
-#pragma unroll
-            for (int e = 0; e < 4; ++e)
-#pragma unroll
-                for (int j = 0; j < DP; ++j) rec[128 * h + DP * (4 * grp + e) + j] = acc[h * DP + j][e] * kUnscale;
-        if (grp == 0) {
-            rec[HD] = m;
-            rec[HD + 1] = l;
         }
+    };
+    uint32_t top = 0;
+#pragma unroll
+    for (int n = 0; n < NT; ++n)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) top = max(top, __float_as_uint(acc[n][e]) & 0x7fffffffu);
+    store();
+    // An infinite V times the parts of p makes NaN (the lower parts are 0 or of
+    // either sign).  Where a sum is not finite, this wavefront takes all of the
+    // split's keys again, now with f32 matrix products of the widened V and
+    // whole p.  The registers of this rare walk are apart from the first's: a
+    // second walk before the merge moved every accumulator (0.5 us a launch).
+    if (__builtin_expect(__any(top >= 0x7f800000u), 0)) {
+        way = 0;
+        ways = 1;
+        clear();
+        for (uint32_t n = 0; pair_block(blk0, n) < blk1; ++n) {
+            if (n % (kWave / 2) == 0) load_table(blk0, n, blk1);
+            cur = pair_at(n);
+            load_k(cur);
+            float p[8];
+            scores(p);
+            load_v(cur);
+            mask(n, p);
+            soften(p);
+#pragma unroll
+            for (int h = 0; h < VH; ++h)
+#pragma unroll
+                for (int j = 0; j < DP; ++j)
+#pragma unroll
+                    for (int i = 0; i < 8; ++i) {
+                        const uint32_t w = vr[i][h][j / 2];
+                        f32x4 &d = acc[h * DP + j];
+                        d = __builtin_amdgcn_mfma_f32_16x16x4f32(C::widen(j % 2 ? w >> 16 : w), p[i], d, 0, 0, 0);
+                    }
+        }
+        l += __shfl_xor(l, 16, kWave);
+        l += __shfl_xor(l, 32, kWave);
+        store();
     }
 }
 

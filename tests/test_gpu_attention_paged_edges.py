@@ -2,7 +2,7 @@
 block, a pair of blocks, a round of the four wavefronts' pairs and a split;
 rows that finish in one split beside rows that need several; walks long enough
 to reload the block-table lanes; windows across splits; non-finite stale bytes
-past a row's length and absent blocks.
+past a row's length and absent blocks; infinite values in attended keys.
 
 Tolerance as in test_gpu_attention.py: 2e-5 of the row's largest |V| plus an
 ulp of the output."""
@@ -87,3 +87,33 @@ def test_stale_bytes_and_absent_blocks(ops, dev, kind, bad, length):
 
         ref = oracle.attention_f32kv(q, nh, nkv, hd, rows(0), rows(1), 0, len(keep))
         check(got, ref, v16, "f32", "absent block")
+
+
+@pytest.mark.parametrize("workspace", ["auto", None])
+@pytest.mark.parametrize("kind,inf", [("f16", 0x7C00), ("bf16", 0x7F80)])
+@pytest.mark.parametrize("nh,nkv,hd", [(8, 2, 64), (32, 2, 128), (4, 1, 256)])
+def test_infinite_value_of_an_attended_key(ops, dev, nh, nkv, hd, kind, inf, workspace):
+    """+inf and -inf in V reach the dims they stand in with their sign, both in
+    one dim make NaN, and every other dim is what it is without them."""
+    rng = np.random.default_rng(hd + nkv)
+    lengths, stride = [1, 20, 600, 1300], nkv * hd
+    q, arena, table, n_logical, bb, v16 = make_case(rng, lengths, nh, nkv, hd, kind)
+    a16 = arena.view(np.uint16).reshape(-1, bb // 2)
+    table2 = table.reshape(len(lengths), n_logical)
+    for r, n in enumerate(lengths):
+        def put(t, dim, bits):
+            a16[table2[r, t // 16], (16 + t % 16) * stride + dim] = bits
+
+        put(0, 3, inf)
+        put(n - 1, hd - 1, inf | 0x8000)
+        put(n // 2, stride - 2, inf)  # the last KV head
+        if n > 1:
+            put(0, hd // 2, inf)
+            put(n - 1, hd // 2, inf | 0x8000)
+    got, _ = run_gpu(ops, dev, q, "f32", "f32", arena, table, n_logical, bb, lengths, nh, nkv, hd, kind,
+                     workspace=workspace)
+    ref = _ref(q, nh, nkv, hd, lengths, arena, table, n_logical, bb, kind)
+    off = ~np.isfinite(ref)
+    assert np.isinf(ref).any() and np.isnan(ref).any()
+    assert np.array_equal(np.where(off, got, 0.0), np.where(off, ref, 0.0), equal_nan=True)
+    check(np.where(off, 0.0, got), np.where(off, 0.0, ref), v16, "f32", "finite dims")

@@ -17,22 +17,24 @@
 // (as up to 16 head slots), so every K/V byte is read once.  Both products of a
 // pair of blocks (2 x 16 tokens) run on the matrix cores:
 //  * S^T = K . Q^T by v_mfma_f32_16x16x32: A = a block's K rows (lane = token
-//    lane % 16, dims 32c + 8 (lane / 16) .. +7 of step c), B = q.  q is split
-//    into f16 high and low parts (two MFMAs per step), so the products with
-//    the f16 cache are exact and the f32 accumulation carries q to ~2^-22
-//    relative; a bf16 cache uses bf16 MFMAs with a three-way split.
+//    lane % 16, dims 32c + 8 (lane / 16) .. +7 of step c), B = q.  For an f16
+//    cache q is split into f16 high and low parts (two MFMAs per step), which
+//    hold f16 values whole and f32 ones to 2^-23 relative where the low part
+//    is normal (|q| above 2^-2), to 2^-25 absolute below; |q| above 65504
+//    overflows.  A bf16 cache uses bf16 MFMAs and three parts: all 24 bits.
 //  * Lane (head slot lane % 16, group lane / 16) then owns the scores of
 //    tokens 4 group .. +3 of each block, which is the layout the second
 //    product takes its B operand in, so the online softmax runs in f32 with
 //    its maximum, rescaling factor and sum per lane, and nothing goes through
 //    LDS.
-//  * out^T = V^T . P^T: the probabilities split as q is (f16 parts after a
-//    scaling by 2^14, so that small ones keep their bits: two parts hold p to
-//    2^-24 relative, three bf16 parts the same), A = V^T assembled from the
-//    lanes' row pieces by byte permutes, f32 accumulation.  The lower parts of
-//    q and p are summed apart from the first, which costs nothing and takes
-//    the error against 64 bits from 0.9 .. 1.15 times that of f32 sums on the
-//    vector ALUs to 0.55 .. 1.05 times.
+//  * out^T = V^T . P^T: the probabilities in three parts, A = V^T assembled
+//    from the lanes' row pieces by byte permutes, f32 accumulation.  Three bf16
+//    parts hold all 24 bits.  The f16 parts do so down to p = 2^-28, to 2^-52
+//    absolute below, since p is scaled by 2^15 and the second and third part
+//    by 2^12 more; their sum is folded in by one FMA.  (Two parts kept 2^-23
+//    and 2^-39, and took 0.2 us less for one row of 64 keys, 0.3 of 27.5 for
+//    32768, 1 of 37 for 256 rows of 16 .. 256.)  The lower parts of q and p are
+//    summed apart from the first, which keeps their bits.
 // The next pair's K is requested once Q.K has read the registers, its V once
 // P.V has.
 //
@@ -88,8 +90,9 @@ struct PagedGeom {
 // Cache element policies: the matrix-core type and the splitting of an f32
 // operand into kParts of them.
 struct CacheF16 {
-    static constexpr int kParts = 2;
-    static constexpr float kPScale = 16384.0f;  // probabilities times this are split
+    static constexpr int kParts = 2, kPParts = 3;
+    static constexpr float kPScale = 32768.0f;  // probabilities times this are split,
+    static constexpr float kPLower = 4096.0f;   // the parts after the first times this more
     // Two values rounded to nearest even and packed; the remainders replace them.
     __device__ static uint32_t part(float &x, float &y) {
         typedef _Float16 half2_t __attribute__((ext_vector_type(2)));
@@ -108,8 +111,8 @@ struct CacheF16 {
 };
 
 struct CacheBF16 {
-    static constexpr int kParts = 3;
-    static constexpr float kPScale = 1.0f;
+    static constexpr int kParts = 3, kPParts = 3;
+    static constexpr float kPScale = 1.0f, kPLower = 1.0f;
     __device__ static uint32_t part(float &x, float &y) {
         typedef __bf16 bf2_t __attribute__((ext_vector_type(2)));
         bf2_t h;
@@ -127,16 +130,19 @@ struct CacheBF16 {
     }
 };
 
-// v[0..7] as kParts operands.
-template <typename C>
-__device__ __forceinline__ void split8(const float (&v)[8], u32x4 (&o)[C::kParts]) {
+// v[0..7] as N operands, the first remainder times `lower`.
+template <typename C, int N>
+__device__ __forceinline__ void split8(const float (&v)[8], float lower, u32x4 (&o)[N]) {
     float rem[8];
 #pragma unroll
     for (int i = 0; i < 8; ++i) rem[i] = v[i];
 #pragma unroll
-    for (int p = 0; p < C::kParts; ++p)
+    for (int p = 0; p < N; ++p)
 #pragma unroll
-        for (int w = 0; w < 4; ++w) o[p][w] = C::part(rem[2 * w], rem[2 * w + 1]);
+        for (int w = 0; w < 4; ++w) {
+            o[p][w] = C::part(rem[2 * w], rem[2 * w + 1]);
+            if (p == 0) rem[2 * w] *= lower, rem[2 * w + 1] *= lower;
+        }
 }
 
 // Keys [lo, seq) of a row: cache blocks [first, last) and how many of the
@@ -287,7 +293,7 @@ __global__ __launch_bounds__(kWave * kDecodeWaves, HD == 64 && C::kParts == 2 ? 
             if (!hv)
 #pragma unroll
                 for (int e = 0; e < 8; ++e) v[e] = 0.0f;
-            split8<C>(v, qb[c]);
+            split8<C>(v, 1.0f, qb[c]);
         }
     }
 
@@ -364,8 +370,8 @@ __global__ __launch_bounds__(kWave * kDecodeWaves, HD == 64 && C::kParts == 2 ? 
         load_k(next);
         mask(n, p);
         soften(p);
-        u32x4 pb[C::kParts];
-        split8<C>(p, pb);
+        u32x4 pb[C::kPParts];
+        split8<C>(p, C::kPLower, pb);
 #pragma unroll
         for (int h = 0; h < VH; ++h)
 #pragma unroll
@@ -378,7 +384,14 @@ __global__ __launch_bounds__(kWave * kDecodeWaves, HD == 64 && C::kParts == 2 ? 
                 // the pair's sum by itself, smallest part first, then once onto the running one
                 f32x4 t = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
-                for (int x = C::kParts - 1; x >= 0; --x) t = C::mfma(a, pb[x], t);
+                for (int x = C::kPParts - 1; x > 0; --x) t = C::mfma(a, pb[x], t);
+                if constexpr (C::kPLower == 1.0f) {
+                    t = C::mfma(a, pb[0], t);
+                } else {
+                    const f32x4 t0 = C::mfma(a, pb[0], f32x4{0.0f, 0.0f, 0.0f, 0.0f});
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) t[e] = __builtin_fmaf(t[e], 1.0f / C::kPLower, t0[e]);
+                }
                 acc[h * DP + j] += t;
             }
         __builtin_amdgcn_sched_barrier(0);

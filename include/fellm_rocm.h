@@ -259,9 +259,12 @@ int fellm_rocm_matvec_kquant(const void *w, uint32_t w_dtype, uint32_t rows, uin
  * partial sums (used when batch * n_kv_heads is small or max_seq large;
  * 16-byte aligned for the fastest combine); with a null or short workspace
  * every (row, KV head) runs in one workgroup.
- * Products with the cache run on the matrix cores and are exact (q and the
- * probabilities are split into 16-bit parts); accumulation, exp and the
- * softmax run in f32.
+ * Products with the cache run on the matrix cores with q and the probabilities
+ * split into 16-bit parts; accumulation, exp and the softmax run in f32.  With
+ * a bf16 cache the parts hold every bit.  With an f16 cache f16 q is held
+ * whole, f32 and bf16 q to 2^-23 relative (2^-25 absolute where |q| < 1/4; |q|
+ * above 65504 overflows) and a probability whole from 2^-28, to 2^-52 absolute
+ * below.  An infinite V gives the infinity or NaN that whole products give.
  */
 uint64_t fellm_rocm_paged_attention_workspace(uint32_t batch, uint32_t n_heads, uint32_t n_kv_heads,
                                               uint32_t head_dim, uint32_t max_seq);

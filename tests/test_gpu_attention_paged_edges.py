@@ -117,3 +117,32 @@ def test_infinite_value_of_an_attended_key(ops, dev, nh, nkv, hd, kind, inf, wor
     assert np.isinf(ref).any() and np.isnan(ref).any()
     assert np.array_equal(np.where(off, got, 0.0), np.where(off, ref, 0.0), equal_nan=True)
     check(np.where(off, 0.0, got), np.where(off, 0.0, ref), v16, "f32", "finite dims")
+
+
+@pytest.mark.parametrize("kind", ["f16", "bf16"])
+@pytest.mark.parametrize("hd", [64, 128, 256])
+def test_small_probabilities_keep_their_bits(ops, dev, hd, kind):
+    """Two keys a row: one of score 0 and V = 0, one of score -x with every V.
+    The output is then p v / (1 + p) with p = exp(-x) down to 2^-29, and shows
+    the bits that p is held to.
+
+    Tolerance, relative: exp takes x log2(e) rounded, an error of |x| 2^-23 in
+    p, and four more roundings of 2^-23 at most (exp itself, the sum, the
+    reciprocal, the products)."""
+    rng = np.random.default_rng(hd)
+    x = np.arange(0, 20.5, 0.25, dtype=np.float32)  # exact in both types
+    rows = x.size
+    k = np.zeros((rows, 2, hd), np.float32)
+    k[:, 1, 0] = -x
+    v = np.zeros((rows, 2, hd), np.float32)
+    v[:, 1] = rng.normal(size=(rows, hd))
+    from test_oracle_attention import build_cache
+
+    arena, table, n_logical, bb, _, v16 = build_cache(rng, list(k), list(v), kind=kind)
+    q = np.zeros((rows, hd), np.float32)
+    q[:, 0] = 1.0
+    got, _ = run_gpu(ops, dev, q, "f32", "f32", arena, table, n_logical, bb, [2] * rows, 1, 1, hd, kind, scale=1.0)
+    p = np.exp(-x.astype(np.float64))[:, None]
+    ref = p / (1.0 + p) * np.stack([r[1] for r in v16])
+    err = np.abs(got - ref) / np.maximum(np.abs(ref), 1e-30)
+    assert np.all(err <= ((x + 4) * 2.0 ** -23)[:, None]), (err.max(1) / ((x + 4) * 2.0 ** -23)).max()

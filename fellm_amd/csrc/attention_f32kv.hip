@@ -71,6 +71,7 @@ struct F32kvArgs {
     // 2: keys within `window` of the row index (all when window == 0).
     uint32_t row_mode, window;
     uint32_t head_major;  // q and out are [head][row][d] instead of [row][head][d]
+    uint32_t out_vec;     // out is 16-byte aligned
 };
 
 // Keys [lo, hi) of the first pair that query row `row` attends.
@@ -368,7 +369,14 @@ __global__ __launch_bounds__(NW *kWave) void attention_f32kv_kernel(F32kvArgs a)
                 float r[VW];
 #pragma unroll
                 for (int x = 0; x < VW; ++x) r[x] = l > 0.0f ? acc[h * VW + x][e] * inv : 0.0f;
-                if (FULL || d < hd) store_f32<F32, VW>(a.out + qoff + d, r);
+                if (FULL || d < hd) {
+                    if (a.out_vec) {
+                        store_f32<F32, VW>(a.out + qoff + d, r);
+                    } else {
+#pragma unroll
+                        for (int x = 0; x < VW; ++x) a.out[qoff + d + x] = r[x];
+                    }
+                }
             }
     }
 }
@@ -391,11 +399,14 @@ int launch_f32kv(const F32kvArgs &a, hipStream_t st) {
 
 // A quarter of the output dims per workgroup, and eight key ways, while one
 // slot tile per workgroup leaves three CUs in four idle (the copies of Q.K
-// then cost idle CUs only).
+// then cost idle CUs only).  Not with out == q: the four workgroups of a slot
+// tile read the same q, which the first to end would overwrite; one workgroup
+// reads its q before its first barrier and writes after its last.
 template <int HD>
 int choose_f32kv(const F32kvArgs &a, hipStream_t st) {
     const uint64_t slots = (uint64_t)a.rows * (a.n_heads / a.n_kv);
-    if (a.n_kv * ((slots + 15) / 16) * 4 <= (uint64_t)cu_count()) return launch_f32kv<HD, HD / 64, 8>(a, st);
+    if (a.q != a.out && a.n_kv * ((slots + 15) / 16) * 4 <= (uint64_t)cu_count())
+        return launch_f32kv<HD, HD / 64, 8>(a, st);
     return launch_f32kv<HD, HD / 16, 4>(a, st);
 }
 
@@ -414,7 +425,7 @@ int attention_f32kv_common(const float *q, float *out, uint32_t rows, uint32_t n
     if (rows == 0) return FELLM_OK;
     if (!(scale > 0.0f)) scale = 1.0f / sqrtf((float)head_dim);
     F32kvArgs a{q, out, k1, v1, k2, v2, rows, n_heads, n_kv_heads, head_dim, begin1, end1, n2, scale, row_mode,
-                window, head_major};
+                window, head_major, aligned_to(out, 16)};
     hipStream_t st = as_stream(stream);
     if (head_dim <= 64) return choose_f32kv<64>(a, st);
     if (head_dim <= 128) return choose_f32kv<128>(a, st);

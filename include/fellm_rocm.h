@@ -287,7 +287,9 @@ int fellm_rocm_paged_attention(const void *q, uint32_t q_dtype, void *out, uint3
  * (k2, v2): out = softmax(q . k * scale) . v, scale <= 0 meaning
  * 1/sqrt(head_dim); query head h uses KV head h / (n_heads / n_kv_heads).
  * No keys gives a zero row.  head_dim % 4 == 0, head_dim <= 256,
- * (n_heads / n_kv_heads) * head_dim <= 2048, 16-byte aligned buffers.
+ * (n_heads / n_kv_heads) * head_dim <= 2048; q, k1, v1, k2 and v2 16-byte
+ * aligned (out too for vector stores; 4 bytes suffice).  out may be q itself
+ * and must not overlap q otherwise, nor k1, v1, k2 or v2.
  * Accumulation and the softmax run in f32 with the device exp.
  */
 int fellm_rocm_attention_f32kv(const float *q, float *out, uint32_t rows, uint32_t n_heads, uint32_t n_kv_heads,
@@ -304,6 +306,7 @@ int fellm_rocm_attention_f32kv(const float *q, float *out, uint32_t rows, uint32
  * `window` of them when window > 0; kv_len >= query_len).  causal == 0: keys
  * within `window` of i (|i - j| < window), every key when window == 0.
  * scale <= 0 means 1/sqrt(head_dim).  Softmax exp is the glibc-exact expf.
+ * Alignment and overlap as for fellm_rocm_attention_f32kv.
  */
 int fellm_rocm_attention_f32kv_rows(const float *q, float *out, uint32_t query_len, uint32_t n_heads,
                                     uint32_t n_kv_heads, uint32_t head_dim, const float *k, const float *v,

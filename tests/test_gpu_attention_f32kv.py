@@ -1,8 +1,8 @@
 """Matrix-core attention over contiguous f32 K/V at the edges of its tiles:
 head dims below, at and between the compiled ones, slot counts around 16, key
 counts around a tile and a workgroup's round of tiles, both output splits (a
-quarter of the dims per workgroup, and all of them), and non-finite V rows that
-only some query rows attend.
+quarter of the dims per workgroup, and all of them), non-finite V rows that
+only some query rows attend, an output in place of q and one aligned to 4 bytes.
 
 Tolerance as in the other attention tests: 2e-5 of the largest |V| (f32 sums
 of at most 1200 products in another order, exp within an ulp) plus an ulp."""
@@ -85,3 +85,33 @@ def test_canvas_edges(rows, past):
     ref = oracle.attention_f32kv(q, nh, nkv, hd, k, v, 0, past, ck, cv, rows)
     assert np.abs(out.cpu().numpy() - ref).max() <= 2e-5 * max(np.abs(v).max(), np.abs(cv).max()) + \
         np.abs(ref).max() * 2.0 ** -23
+
+
+@pytest.mark.parametrize("hd", [60, 64, 128, 256])
+@pytest.mark.parametrize("rows", [1, 7, 200])
+def test_out_in_place_and_at_4_bytes(rows, hd):
+    """The same bits whether out stands apart, in place of q or one f32 past a
+    16-byte boundary.  In place takes the kernel with all dims in a workgroup,
+    whose sums run over other tiles: there the tolerance of this file."""
+    from fellm_amd import _lib
+
+    nh, nkv, keys = 8, 2, 500
+    rng = np.random.default_rng(rows + hd)
+    q, k, v = _inputs(rng, nh, nkv, hd, rows, keys)
+    ref = oracle.attention_f32kv(q.reshape(rows, nh * hd), nh, nkv, hd, k, v, 0, keys).reshape(-1)
+    kd, vd = torch.from_numpy(k).cuda(), torch.from_numpy(v).cuda()
+
+    def run(qd, out):
+        rc = _lib.lib().fellm_rocm_attention_f32kv(qd.data_ptr(), out.data_ptr(), rows, nh, nkv, hd, kd.data_ptr(),
+                                                   vd.data_ptr(), 0, keys, None, None, 0, 0.0,
+                                                   torch.cuda.current_stream().cuda_stream)
+        assert rc == 0, rc
+        return out.cpu().numpy()
+
+    qd = torch.from_numpy(q).cuda()
+    apart = run(qd, torch.empty_like(qd))
+    wide = torch.full((q.size + 2,), 7.0, device="cuda")
+    assert np.array_equal(run(qd, wide[1:-1]), apart)
+    assert wide[0].item() == 7.0 and wide[-1].item() == 7.0
+    for got in (apart, run(qd, qd)):
+        assert np.abs(got - ref).max() <= 2e-5 * np.abs(v).max() + np.abs(ref).max() * 2.0 ** -23

@@ -67,6 +67,34 @@ def test_rows_nonfinite_value_stays_with_its_rows(causal, window, bad):
     assert np.abs(got[~hit] - clean[~hit]).max() <= 2e-5 * np.abs(v).max()
 
 
+@pytest.mark.parametrize("hd", [60, 64, 68, 128, 132, 256])
+@pytest.mark.parametrize("ql", [6, 150])
+@pytest.mark.parametrize("causal,window", [(True, 0), (False, 9)])
+@pytest.mark.parametrize("bad", [np.inf, np.nan])
+def test_nonfinite_key_of_some_rows_in_every_kernel(hd, ql, causal, window, bad):
+    """The key-by-key walk in both output splits and every padding of the head
+    dim: bad V dims in each quarter of the output, and a bad K row, all of one
+    key that half of the rows attend."""
+    nh, nkv, kvl = 8, 2, 170
+    rng = np.random.default_rng(hd + ql)
+    q, k, v = _inputs(rng, nh, nkv, hd, ql, kvl)
+    at = kvl - ql // 2 - 1 if causal else ql // 2 + 8
+    dims = [1, hd // 3, hd // 2 + 1, hd - 2]
+    k2, v2 = k.copy(), v.copy()
+    k2[at, 3] = bad  # KV head 0
+    v2[at, [hd + d for d in dims]] = bad  # KV head 1
+    clean = _rows(q, k, v, nh, nkv, hd, ql, kvl, causal, window).reshape(nh, ql, hd)
+    got = _rows(q, k2, v2, nh, nkv, hd, ql, kvl, causal, window).reshape(nh, ql, hd)
+    row = np.arange(ql)
+    sees = at <= kvl - ql + row if causal else np.abs(row - at) < window
+    assert sees.any() and not sees.all()
+    hit = np.zeros((nh, ql, hd), bool)
+    hit[np.ix_(np.arange(nh // nkv, nh), sees, dims)] = True
+    assert np.all(~np.isfinite(got[hit]))
+    hit[:nh // nkv, sees] = True  # a bad score: whatever its row then holds
+    assert np.abs(got[~hit] - clean[~hit]).max() <= 2e-5 * np.abs(v).max()
+
+
 @pytest.mark.parametrize("rows,past", [(16, 1), (33, 47), (80, 1000)])
 def test_canvas_edges(rows, past):
     from fellm_amd import _lib

@@ -978,6 +978,7 @@ int launch_emb(const void *table, uint64_t vocab, uint32_t dim, const uint32_t *
     FELLM_EMB(2, true)
     FELLM_EMB(4, true)
     FELLM_EMB(8, true)
+    if constexpr (D::OUT == 4) FELLM_EMB(16, true)  // f32 rows of 8192 .. 16384 in parts of 4
 #undef FELLM_EMB
     return FELLM_ERR_SHAPE;
 }

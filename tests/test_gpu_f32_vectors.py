@@ -1,6 +1,6 @@
 """f32 ops in 4-element vectors and bf16 gathers rounded in pairs: lengths
 around a vector and a workgroup, buffers aligned to 16 but not 32 bytes and to 4
-bytes only, rows of every register layout of RMSNorm, NaN payloads.  Bit-exact
+bytes only, rows of every register layout of RMSNorm and of the fused f32 gather, NaN payloads.  Bit-exact
 against the oracle; RMSNorm within 1e-5 (its sum runs in another order)."""
 from __future__ import annotations
 
@@ -80,6 +80,23 @@ def test_kquant_gather_rows(ops, qt, code, n, blocks, kind):
     d = ref.astype(np.float64)
     yr = d / np.sqrt((d * d).mean(-1, keepdims=True) + 1e-6)
     assert np.abs(y.double().cpu().numpy() - yr).max() <= (1e-5 if kind == "f32" else 2.0 ** -8) * np.abs(yr).max()
+
+
+@pytest.mark.parametrize("n", [3, 700])
+@pytest.mark.parametrize("dim", [1000, 4096, 8192, 8200, 8448, 16384])
+def test_dense_f32_gather_and_norm(ops, dim, n):
+    """Rows up to the longest that the fused f32 norm takes, few and many."""
+    rng = np.random.default_rng(dim + n)
+    table = rng.normal(size=(40, dim)).astype(np.float32)
+    ids = rng.integers(0, 40, size=n, dtype=np.uint32)
+    w = rng.normal(1.0, 0.1, size=dim).astype(np.float32)
+    tab, idd, wd = torch.from_numpy(table).cuda(), torch.from_numpy(ids.view(np.int32)).cuda(), torch.from_numpy(w).cuda()
+    got = ops.embedding(tab, idd, out_dtype=torch.float32)
+    h, y = ops.embedding_rmsnorm(tab, idd, wd, 1e-6, out_dtype=torch.float32)
+    assert np.array_equal(_bits(got), table[ids].view(np.uint32)) and np.array_equal(_bits(h), _bits(got))
+    d = table.astype(np.float64)
+    ref = (d / np.sqrt((d * d).mean(-1, keepdims=True) + 1e-6) * w)[ids]
+    assert np.abs(y.cpu().numpy() - ref).max() <= 1e-5 * np.abs(ref).max()
 
 
 def test_bf16_gather_keeps_nan_payloads(ops):

@@ -686,10 +686,13 @@ __global__ __launch_bounds__(NW * kWave) void kquant_gemv_kernel(const uint8_t *
 // x slice from LDS for every 32 blocks, at an eight-way bank conflict, and
 // folded its row in a single lane: 8192 x 28672 Q4_K 41.2 -> 28.4 us, Q6_K 58.6
 // -> 43.3, 4096 x 14336 Q4_K 13.0 -> 11.3, 5120 x 13824 20.0 -> 13.2; with 8
-// wavefronts per workgroup instead of 16 31.1, 46.0, 11.5 and 13.5.)  The block values of kFoldRows rows per
-// group collect in LDS; after a barrier one wavefront, another for every
-// batch, folds all of them, a lane per (row, matrix), while the others go on
-// into the second fold buffer.
+// wavefronts per workgroup instead of 16 31.1, 46.0, 11.5 and 13.5.)  The
+// workgroup has more wavefronts than the launch's passes * groups: the others
+// take their part of x's quantization and end (256 x 16384 Q4_K in workgroups
+// of two wavefronts 16.3 us, with 14 more for x 7.1).  The block values of kFoldRows
+// rows per group collect in LDS; after a barrier one wavefront, another for
+// every batch, folds all of them, a lane per (row, matrix), while the others go
+// on into the second fold buffer.
 constexpr uint32_t kFoldRows = 4;
 constexpr uint32_t gemv_pass_lds(uint32_t nb, uint32_t passes, uint32_t groups, uint32_t mats, uint32_t stage) {
     const uint32_t nbp = (nb + 3) & ~3u;
@@ -711,7 +714,8 @@ __global__ __launch_bounds__(MAXW * kWave) void kquant_gemv_passes(const uint8_t
     const uint32_t nbp = (nb + 3) & ~3u;
     const uint32_t pass = wave % passes, group = wave / passes, waves = passes * groups;
     const uint32_t per = (nb + passes - 1) / passes, first = pass * per;
-    const uint32_t mine = first < nb ? (nb - first < per ? nb - first : per) : 0;
+    const bool helper = wave >= waves;  // prepares x and ends
+    const uint32_t mine = first < nb && !helper ? (nb - first < per ? nb - first : per) : 0;
     const uint32_t batch_floats = groups * kFoldRows * kMats * nbp;
     uint8_t *stage = reinterpret_cast<uint8_t *>(xl.fold + 2 * batch_floats) + wave * kStagePerWave<GW, UW, FUSED>;
     uint8_t *ustage = stage + 1024 * kChunks<GW>;
@@ -723,7 +727,7 @@ __global__ __launch_bounds__(MAXW * kWave) void kquant_gemv_passes(const uint8_t
     const uint32_t steps = (rows + gridDim.x * groups - 1) / (gridDim.x * groups);
     auto range = [&](uint32_t n, uint32_t rb, uint32_t kb, uint32_t &b0, uint32_t &b1) {
         const uint32_t r = row_of(n, group);
-        b0 = r < rows ? r * rb + first * kb : 0;
+        b0 = r < rows && !helper ? r * rb + first * kb : 0;
         b1 = r < rows ? b0 + mine * kb : 0;
     };
 
@@ -759,6 +763,7 @@ __global__ __launch_bounds__(MAXW * kWave) void kquant_gemv_passes(const uint8_t
     if (threadIdx.x < 32) tab_lds[threadIdx.x] = tab_v;
     x_finish<PREQ>(x, nb, xl, gemv_smem, xf);
     barrier();
+    if (helper) return;  // an ended wavefront takes no part in the barriers below
     const bool on = slot < mine;
     XHalf xh;
     load_x(xl, on ? first + slot : 0, h, xh);
@@ -917,7 +922,11 @@ int launch_gemv(const void *gw, const void *uw, const void *x, float *out, uint3
             // than give every CU a workgroup (each quantizes x: 2048 x 9472
             // Q4_K 7.6 us in 256 workgroups, 9.6 in 512 half as wide); among
             // those of at least half as many, the one that leaves the fewest
-            // group slots of the last step empty.
+            // group slots of the last step empty.  What one step of more than
+            // half of the wavefronts would take goes in two steps of half as
+            // many, the second's weights on their way during the first: 2048 x
+            // 16384 Q4_K 10.1 -> 9.3 us, Q6_K 14.1 -> 12.3, from a blob 8.8 ->
+            // 7.6 and 13.1 -> 11.0; 1024 x 28672 Q4_K 13.3 -> 12.4.
             constexpr int MAXW = FUSED ? 8 : 16;
             const uint32_t passes = (nb + 31) / 32;
             auto lds_of = [&](uint32_t g) { return gemv_pass_lds(nb, passes, g, mats, kStagePerWave<GW, UW, FUSED>); };
@@ -931,14 +940,19 @@ int launch_gemv(const void *gw, const void *uw, const void *x, float *out, uint3
                 const uint32_t all = (uint32_t)cu_count() * (per_cu ? per_cu : 1), need = (n + g - 1) / g;
                 return need < all ? need : all;
             };
-            uint32_t groups = most;
+            const bool two_steps = !FUSED && one_step <= most && passes * one_step > MAXW / 2;
+            uint32_t groups = two_steps ? (one_step + 1) / 2 : most;
             uint64_t best = ~0ull;
-            for (uint32_t g = most; 2 * g >= most && g > 0; --g) {
+            for (uint32_t g = most; !two_steps && 2 * g >= most && g > 0; --g) {
                 const uint64_t per_step = (uint64_t)grid_of(g) * g, slots = (n + per_step - 1) / per_step * per_step;
                 if (slots < best) best = slots, groups = g;
             }
-            FELLM_LAUNCH((kquant_gemv_passes<GW, UW, FUSED, PREQ, MAXW>), dim3(grid_of(groups)),
-                         dim3(passes * groups * kWave), lds_of(groups), s, g, u, x, out + r0, n, nb, passes, groups);
+            // A blob's copy wants fewer helpers: 700 x 25600 Q6_K 10.7 us with 8
+            // wavefronts in all, 11.1 with 16; 256 x 16384 7.0 with 2, 5.7 with 16.
+            const uint32_t waves = std::max(passes * groups, PREQ ? 8u : (uint32_t)MAXW);
+            const uint32_t grid = two_steps ? (uint32_t)cu_count() : grid_of(groups);
+            FELLM_LAUNCH((kquant_gemv_passes<GW, UW, FUSED, PREQ, MAXW>), dim3(grid), dim3(waves * kWave), lds_of(groups),
+                         s, g, u, x, out + r0, n, nb, passes, groups);
         }
         const int rc = launch_status();
         if (rc != FELLM_OK) return rc;

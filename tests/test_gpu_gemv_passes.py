@@ -49,3 +49,17 @@ def test_gate_up_passes(ops, gq, uq, rows, nb):
     ref = oracle.gate_up_swiglu(CODE[gq], g, CODE[uq], u, rows, nb * 256, x).view(np.uint32)
     assert np.array_equal(_bits(ops.gate_up_swiglu(gd, ud, xd, qtype=gq, up_qtype=uq)), ref)
     assert np.array_equal(_bits(ops.gate_up_swiglu_q8k(gd, ud, ops.quantize_q8k(xd), qtype=gq, up_qtype=uq)), ref)
+
+
+@pytest.mark.parametrize("qt", ["q4k", "q5k", "q6k"])
+@pytest.mark.parametrize("rows,nb", [(256, 64), (257, 40), (1024, 64), (1025, 64), (1536, 33), (2047, 64), (2049, 64),
+                                     (1280, 80), (768, 129), (512, 192)])
+def test_wavefronts_for_x_and_two_steps(ops, qt, rows, nb):
+    """Launches whose workgroups hold wavefronts that only prepare x, on both
+    sides of the choice between one step and two, the last rows uneven."""
+    test_matvec_passes(ops, qt, rows, nb)
+
+
+@pytest.mark.parametrize("rows,nb", [(200, 40), (256, 64), (257, 80), (300, 112)])
+def test_gate_up_wavefronts_for_x(ops, rows, nb):
+    test_gate_up_passes(ops, "q4k", "q6k", rows, nb)

@@ -173,16 +173,17 @@ __device__ __forceinline__ float rows_max(float v) {
 }
 
 // Q: query activation policy, O: output policy, C: cache policy, HD: head
-// dim (64, 128 or 256).  rec_heads: head slots of a partial record.  early:
+// dim (64, 128 or 256), W: wavefronts.  solo: pairs of blocks that one
+// wavefront takes alone.  rec_heads: head slots of a partial record.  early:
 // the first blocks are requested before the row length is known.
-template <typename Q, typename O, typename C, int HD>
-__global__ __launch_bounds__(kWave * kDecodeWaves, HD == 64 && C::kParts == 2 ? 4 : 1) void paged_decode_kernel(const typename Q::T *__restrict__ q,
+template <typename Q, typename O, typename C, int HD, uint32_t W>
+__global__ __launch_bounds__(kWave *W, HD == 64 && C::kParts == 2 ? 4 : 1) void paged_decode_kernel(const typename Q::T *__restrict__ q,
                                                              typename O::T *__restrict__ out,
                                                              float *__restrict__ part, const uint32_t *__restrict__ lens,
                                                              PagedGeom geo, uint32_t batch, uint32_t n_heads,
                                                              uint32_t n_kv, float scale, uint32_t causal,
                                                              uint32_t window, uint32_t splits, uint32_t bps,
-                                                             uint32_t rec_heads, uint32_t early) {
+                                                             uint32_t rec_heads, uint32_t early, uint32_t solo) {
     constexpr int NC = HD / 32;               // Q.K steps, and 16-byte K loads per lane and block
     constexpr int DP = HD < 128 ? 4 : 8;      // consecutive dims of a lane's V piece
     constexpr int VH = HD / 16 / DP;          // V pieces per token row
@@ -202,7 +203,7 @@ __global__ __launch_bounds__(kWave * kDecodeWaves, HD == 64 && C::kParts == 2 ? 
     // This wavefront's pairs of blocks: first + 2 (way + ways n), n = 0, 1, ..
     // Lane l holds the physical block (~0: none, or at or past lim) of block
     // l % 2 of pair tab0 + l / 2; a walk of more than 32 pairs reloads.
-    uint32_t tab = ~0u, tab0 = 0, way = wave, ways = kDecodeWaves;
+    uint32_t tab = ~0u, tab0 = 0, way = wave, ways = W;
     auto pair_block = [&](uint32_t first, uint32_t n) { return first + 2 * (way + ways * n); };
     auto load_table = [&](uint32_t first, uint32_t n, uint32_t lim) {
         tab0 = n;
@@ -274,6 +275,12 @@ __global__ __launch_bounds__(kWave * kDecodeWaves, HD == 64 && C::kParts == 2 ? 
     if (s >= (row.splits ? row.splits : 1)) return;
     const uint32_t blk0 = row.first + s * bps;
     const uint32_t blk1 = blk0 + bps < row.last ? blk0 + bps : row.last;
+    // Wavefronts without a pair of blocks end here and take no part in the
+    // barriers below (256 rows of 30 keys, 32/8 heads of 128, in a launch made
+    // for 4096: 23.2 -> 11.5 us).
+    const uint32_t has = (blk1 - blk0 + 1) / 2, live = has <= solo ? 1 : has < W ? has : W;
+    if (wave >= live) return;
+    if (live == 1) ways = 1;
     if (!early) {
         load_table(blk0, 0, blk1);
         cur = pair_at(0);
@@ -404,7 +411,8 @@ __global__ __launch_bounds__(kWave * kDecodeWaves, HD == 64 && C::kParts == 2 ? 
     // Merge the wavefronts pairwise through LDS: [half, 2 half) hand theirs to [0, half).
     constexpr uint32_t kMerge = (NT * 4 + 2) * kWave;  // floats per wavefront
 #pragma unroll
-    for (uint32_t half = kDecodeWaves / 2; half > 0; half /= 2) {
+    for (uint32_t half = W / 2; half > 0; half /= 2) {
+        if (half >= live) continue;  // the same in every live wavefront
         float *rec = merge_lds + (size_t)(wave % half) * kMerge + lane;
         __syncthreads();
         if (wave >= half && wave < 2 * half) {
@@ -416,7 +424,7 @@ __global__ __launch_bounds__(kWave * kDecodeWaves, HD == 64 && C::kParts == 2 ? 
                 for (int e = 0; e < 4; ++e) rec[(2 + n * 4 + e) * kWave] = acc[n][e];
         }
         __syncthreads();
-        if (wave < half) {
+        if (wave < half && wave + half < live) {
             const float mo = rec[0], mn = fmaxf(m, mo);
             const float wa = m > -__builtin_inff() ? __expf(m - mn) : 0.0f;
             const float wb = mo > -__builtin_inff() ? __expf(mo - mn) : 0.0f;
@@ -657,7 +665,9 @@ __global__ __launch_bounds__(kWave) void paged_decode_combine_wave(const float *
 
 // Splits of a row's keys over workgroups.
 //  * Few (row, KV head) pairs: about one workgroup per CU, at least 8 blocks
-//    each (a pair of blocks per wavefront); rows of up to 32 blocks stay whole.
+//    each (a pair of blocks per wavefront); rows of up to 32 blocks stay whole,
+//    at heads of 256 of up to 24 (512 keys 17.5 us whole, 13.4 in four splits).
+//    A window that fits stays whole too (128 of 4096 keys 7.5 -> 6.3 us).
 //    One row at 8 KV heads: 256 keys 6.6 us whole, 8.9 in two splits; 2048 keys
 //    9.9 us in 16 splits, 11.3 in 8; 32768 keys 27.3 in 32, 28.4 in 64.
 //  * Long rows: splits of 128 blocks (2048 keys) while the launch stays within
@@ -665,18 +675,36 @@ __global__ __launch_bounds__(kWave) void paged_decode_combine_wave(const float *
 //    longest rows.  64 rows of 256 .. 4096 keys: 123.7 us against 118.4 with
 //    splits of 64 blocks, but 64 rows of 4096 keys each 194 against 202; 256
 //    rows of 4096 keys 677 us whole, 740 in two splits.
-constexpr uint32_t kSplitTarget = 256, kMinSplitBlocks = 8, kWholeBlocks = 32;
+constexpr uint32_t kSplitTarget = 256, kMinSplitBlocks = 8;
 constexpr uint32_t kLongSplitBlocks = 128, kLongSplitMax = 2048;
-uint32_t choose_splits(uint32_t batch, uint32_t n_kv, uint32_t max_seq) {
+uint32_t whole_blocks(uint32_t head_dim) { return head_dim == 256 ? 24 : 32; }
+uint32_t choose_splits(uint32_t batch, uint32_t n_kv, uint32_t max_seq, uint32_t head_dim) {
     const uint32_t pairs = batch * n_kv;
     const uint32_t blocks = (max_seq + kBlockTokens - 1) / kBlockTokens;
-    if (pairs == 0 || blocks <= kWholeBlocks) return 1;
+    if (pairs == 0 || blocks <= whole_blocks(head_dim)) return 1;
     uint32_t s = (kSplitTarget + pairs - 1) / pairs;
     if (s > blocks / kMinSplitBlocks) s = blocks / kMinSplitBlocks;
     uint32_t by_length = (blocks + kLongSplitBlocks - 1) / kLongSplitBlocks;
     if (by_length > kLongSplitMax / pairs) by_length = kLongSplitMax / pairs;
     if (s < by_length) s = by_length;
     return s < kMaxSplits ? s : kMaxSplits;
+}
+
+// One wavefront a workgroup instead of kDecodeWaves: no merge, and more
+// workgroups on a CU.  Where a pair of blocks is all there is (8 rows of 32
+// keys, 32/8 heads of 128: 4.2 against 4.5 us), and where the (row, KV head)
+// pairs alone fill the chip and no row is long: a row's one wavefront must not
+// outlast the others.  At 256 rows of these heads: 32 keys 8.1 us against 10.4,
+// 100 keys 22.0 and 32.2, 512 keys 79.5 and 82.9, 16 .. 512 53.0 and 52.9, but
+// 16 .. 768 81 and 71.  Heads of 64 turn at half of that (256 rows, 8/8 heads:
+// 16 .. 256 keys 18.2 and 18.6, 16 .. 384 26.1 and 23.5); heads of 256 at twice
+// (128 rows, 16/8 heads: 16 .. 1024 keys 100 and 106, 16 .. 2048 200 and 193),
+// and from half as many pairs (64 rows of 512 keys 43 and 49), where the others
+// gain up to head_dim keys (64 rows of 64 keys 5.9 and 6.8, of 200 12.3 and 11.7).
+bool fills(uint32_t pairs, uint32_t head_dim) { return pairs >= (head_dim == 256 ? 512u : 1024u); }
+bool one_wave(uint32_t pairs, uint32_t blocks, uint32_t bps, uint32_t head_dim) {
+    return blocks <= 2 || (pairs >= 512 && blocks <= head_dim / 16) ||
+           (fills(pairs, head_dim) && bps <= head_dim / 4);
 }
 
 // Launches of at most this many workgroups request their first blocks before
@@ -691,17 +719,30 @@ int launch_decode(const void *q, void *out, uint32_t batch, uint32_t n_heads, ui
                   uint32_t max_seq, float scale, uint32_t causal, uint32_t window, const PagedGeom &geo,
                   float *ws, uint64_t ws_bytes, hipStream_t st) {
     const uint32_t gm = n_heads / n_kv <= 8 ? 8 : 16;
-    uint32_t splits = choose_splits(batch, n_kv, max_seq);
+    const uint32_t blocks = (max_seq + kBlockTokens - 1) / kBlockTokens;
+    // Blocks that a row attends at most: a window's keys start anywhere in a block.
+    const uint32_t held = causal && window
+                              ? (uint32_t)std::min<uint64_t>(blocks, ((uint64_t)window + 2 * kBlockTokens - 2) / kBlockTokens)
+                              : blocks;
+    uint32_t splits = held <= whole_blocks(HD) ? 1 : choose_splits(batch, n_kv, max_seq, HD);
     const uint64_t need = (uint64_t)batch * n_kv * splits * gm * (HD + kRecTail) * 4;
     if (splits > 1 && (!ws || ws_bytes < need)) splits = 1;
-    const uint32_t blocks = (max_seq + kBlockTokens - 1) / kBlockTokens;
     const uint32_t bps = blocks ? (blocks + splits - 1) / splits : 1;
     const uint32_t grid = batch * n_kv * splits;
-    const uint32_t lds = kDecodeWaves / 2 * (HD / 4 + 2) * kWave * sizeof(float);
-    const uint32_t early = !(causal && window) && grid <= kEarlyGrid;
-    FELLM_LAUNCH((paged_decode_kernel<Q, O, C, HD>), dim3(grid), dim3(kWave * kDecodeWaves), lds, st,
-                 static_cast<const typename Q::T *>(q), static_cast<typename O::T *>(out), ws, lens, geo, batch, n_heads,
-                 n_kv, scale, causal, window, splits, bps, gm, early);
+    // Short rows of a launch that fills the chip for long ones (128 rows of 100
+    // keys, 32/8 heads of 128, made for 4096: 20.6 -> 17.6 us).
+    const uint32_t solo = HD < 256 && fills(batch * n_kv, HD) ? 4 : 1;
+    const uint32_t early = !(causal && window) && grid <= kEarlyGrid && solo == 1;
+    auto decode = [&]<uint32_t W>() {
+        const uint32_t lds = W / 2 * (HD / 4 + 2) * kWave * sizeof(float);
+        FELLM_LAUNCH((paged_decode_kernel<Q, O, C, HD, W>), dim3(grid), dim3(kWave * W), lds, st,
+                     static_cast<const typename Q::T *>(q), static_cast<typename O::T *>(out), ws, lens, geo, batch,
+                     n_heads, n_kv, scale, causal, window, splits, bps, gm, early, solo);
+    };
+    if (one_wave(batch * n_kv, held, std::min(bps, held), HD))
+        decode.template operator()<1>();
+    else
+        decode.template operator()<kDecodeWaves>();
     int rc = launch_status();
     if (rc != FELLM_OK || splits == 1) return rc;
     auto combine = [&]<int GM>() {
@@ -720,7 +761,7 @@ int launch_decode(const void *q, void *out, uint32_t batch, uint32_t n_heads, ui
 }
 
 template <typename Q, typename O, typename C>
-int dispatch_hd(uint32_t hd, uint32_t G, const void *q, void *out, uint32_t batch, uint32_t n_heads, uint32_t n_kv,
+int dispatch_hd(uint32_t hd, const void *q, void *out, uint32_t batch, uint32_t n_heads, uint32_t n_kv,
                 const uint32_t *lens, uint32_t max_seq, float scale, uint32_t causal, uint32_t window,
                 const PagedGeom &geo, float *ws, uint64_t ws_bytes, hipStream_t st) {
 #define FELLM_ATT(HDV)                                                                                              \
@@ -741,7 +782,7 @@ extern "C" uint64_t fellm_rocm_paged_attention_workspace(uint32_t batch, uint32_
                                                          uint32_t head_dim, uint32_t max_seq) {
     using namespace fellm;
     if (!n_kv_heads || n_heads % n_kv_heads) return 0;
-    const uint32_t splits = choose_splits(batch, n_kv_heads, max_seq);
+    const uint32_t splits = choose_splits(batch, n_kv_heads, max_seq, head_dim);
     if (splits <= 1) return 0;
     const uint32_t gm = n_heads / n_kv_heads <= 8 ? 8 : 16;
     return (uint64_t)batch * n_kv_heads * splits * gm * (head_dim + kRecTail) * 4;
@@ -764,15 +805,14 @@ extern "C" int fellm_rocm_paged_attention(const void *q, uint32_t q_dtype, void 
     const PagedGeom geo{static_cast<const uint8_t *>(kv->arena), kv->arena_len, kv->block_table, kv->n_block_table,
                         kv->n_logical_blocks, kv->n_layers, kv->layer, kv->block_size, kv->block_bytes, kv->stride};
     hipStream_t st = as_stream(stream);
-    const uint32_t G = n_heads / n_kv_heads;
     if (kv->kv_dtype != FELLM_DTYPE_F16 && kv->kv_dtype != FELLM_DTYPE_BF16) return FELLM_ERR_DTYPE;
     const bool bf = kv->kv_dtype == FELLM_DTYPE_BF16;
 #define FELLM_ATT_QO(QD, QT, OD, OT)                                                                              \
     if (q_dtype == QD && out_dtype == OD)                                                                         \
-        return bf ? dispatch_hd<QT, OT, CacheBF16>(head_dim, G, q, out, batch, n_heads, n_kv_heads, row_lengths,  \
+        return bf ? dispatch_hd<QT, OT, CacheBF16>(head_dim, q, out, batch, n_heads, n_kv_heads, row_lengths,  \
                                                    max_seq, scale, causal, window, geo, workspace, workspace_bytes, \
                                                    st)                                                            \
-                  : dispatch_hd<QT, OT, CacheF16>(head_dim, G, q, out, batch, n_heads, n_kv_heads, row_lengths,   \
+                  : dispatch_hd<QT, OT, CacheF16>(head_dim, q, out, batch, n_heads, n_kv_heads, row_lengths,   \
                                                   max_seq, scale, causal, window, geo, workspace, workspace_bytes,  \
                                                   st);
     FELLM_ATT_QO(FELLM_DTYPE_F32, F32, FELLM_DTYPE_F32, F32)

@@ -2,7 +2,8 @@
 block, a pair of blocks, a round of the four wavefronts' pairs and a split;
 rows that finish in one split beside rows that need several; walks long enough
 to reload the block-table lanes; windows across splits; non-finite stale bytes
-past a row's length and absent blocks; infinite values in attended keys.
+past a row's length and absent blocks; infinite values in attended keys; the
+choice between one and four wavefronts.
 
 Tolerance as in test_gpu_attention.py: 2e-5 of the row's largest |V| plus an
 ulp of the output."""
@@ -146,3 +147,23 @@ def test_small_probabilities_keep_their_bits(ops, dev, hd, kind):
     ref = p / (1.0 + p) * np.stack([r[1] for r in v16])
     err = np.abs(got - ref) / np.maximum(np.abs(ref), 1e-30)
     assert np.all(err <= ((x + 4) * 2.0 ** -23)[:, None]), (err.max(1) / ((x + 4) * 2.0 ** -23)).max()
+
+
+@pytest.mark.parametrize("kind", ["f16", "bf16"])
+@pytest.mark.parametrize("rows,nh,nkv,hd,top", [
+    (3, 8, 2, 64, 32), (3, 4, 1, 256, 33),  # one pair of blocks or more
+    (8, 64, 64, 64, 64), (8, 64, 64, 64, 65), (8, 128, 64, 128, 128), (8, 64, 64, 128, 129),  # 512 (row, KV head) pairs
+    (16, 128, 64, 64, 256), (16, 64, 64, 64, 257), (16, 64, 64, 128, 300), (7, 64, 64, 256, 40), (8, 64, 64, 256, 200)])
+def test_one_or_four_wavefronts(ops, dev, rows, nh, nkv, hd, top, kind):
+    """Both sides of each line of the choice, with rows of 0 to `top` keys and an
+    infinite V in the longest."""
+    rng = np.random.default_rng(top + hd)
+    lengths = [top, 0, 1] + [int(n) for n in rng.integers(1, top + 1, size=rows - 3)]
+    q, arena, table, n_logical, bb, v16 = make_case(rng, lengths, nh, nkv, hd, kind)
+    a16 = arena.view(np.uint16).reshape(-1, bb // 2)
+    a16[table[0], 16 * nkv * hd + 5] = 0xFF80 if kind == "bf16" else 0xFC00  # key 0 of row 0, dim 5: -inf
+    got, _ = run_gpu(ops, dev, q, "f32", "f32", arena, table, n_logical, bb, lengths, nh, nkv, hd, kind)
+    ref = _ref(q, nh, nkv, hd, lengths, arena, table, n_logical, bb, kind)
+    off = ~np.isfinite(ref)
+    assert off.any() and np.array_equal(got[off], ref[off])
+    check(np.where(off, 0.0, got), np.where(off, 0.0, ref), v16, "f32", f"top {top}")

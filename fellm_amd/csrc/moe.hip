@@ -267,8 +267,9 @@ __global__ __launch_bounds__(BLOCK) void moe_scatter_blocks(const uint32_t *__re
     scatter_range(ids, wlo, whi, E, bits, wcur + w * E, order, inv);
 }
 
-// Block count and chunk (a multiple of kDispatchBlock, so each wavefront's
-// quarter is whole rounds) for n assignments.
+// Block count and chunk for n assignments.  The chunk is a multiple of
+// kDispatchBlock, so a quarter of it is whole rounds of 64; a sixteenth may
+// end in a part of one.
 struct DispatchGrid {
     uint32_t nblocks;
     uint64_t chunk;
@@ -306,12 +307,12 @@ __device__ __forceinline__ void store_vec(V *p, const V &v) {
     }
 }
 
-// Bytes from which the expert rows (combine) and the grouped rows (gather) are
-// streamed: half of the 256 MB last-level cache.  Below, a caller's next or
-// previous kernel may find them there.  Measured: combine of 16384 tokens x 8
-// rows of 8 KB 261 -> 225 us in expert order and 231 -> 199 in slot order, of
-// 512 tokens 9.4 -> 10.0 (so it stays plain).
-constexpr uint64_t kStreamBytes = 128ull << 20;
+// Bytes from which the grouped rows (gather) and the expert rows (combine) are
+// streamed: half and three quarters of the 256 MB last-level cache.  Below, a
+// caller's next or previous kernel may find them there.  Measured: gather of
+// 134 MB 37.7 -> 30.7 us; combine of 240 MB 64.3 -> 56.3 us, of 180 MB 47.2 ->
+// 48.7, of 134 MB 39.6 -> 41.9.
+constexpr uint64_t kGatherStreamBytes = 128ull << 20, kCombineStreamBytes = 192ull << 20;
 
 // grouped[i] = x[order[i] / top_k]; an invalid order entry gives a zero row.
 template <typename V>
@@ -390,10 +391,11 @@ __global__ __launch_bounds__(256) void moe_scatter_rows(const uint4 *__restrict_
 // y[t] = y0[t] (or 0) + sum over t's slots of weight * row, one token per
 // block iteration.  EXPERT_ORDER: slots in ascending (expert id, slot), rows
 // expert_out[inv[a]]; otherwise slot order, rows expert_out[a].  Bound by the
-// rows' bytes.  Workgroups of 1024 threads where a row has more than 512
-// vectors (top-4 rows of 16 KB 75.6 -> 67.7 us, top-8 rows of 11.5 KB 337 ->
-// 326), of 512 otherwise (top-8 rows of 8 KB 225 us, 264 with 1024, 240 with
-// 256).
+// rows' bytes.  Workgroups of 512 threads (top-8 rows of 8 KB 225 us, 264 with
+// 1024, 240 with 256), of 1024 where a row has more than 512 vectors and a CU
+// few tokens (512 tokens of top-4 rows of 11.5 KB 6.9 -> 5.4 us, 16 of top-6
+// rows of 20 KB 6.3 -> 5.0; but 2048 22.2 -> 23.9, of 1001 single elements 15.9
+// -> 18.2) or streams (16384 tokens of top-4 rows of 16 KB 246 -> 233).
 template <bool EXPERT_ORDER, int VEC, bool NT>
 __global__ __launch_bounds__(1024) void moe_combine_rows(const float *y0, const float *__restrict__ expert_out,
                                                         const uint32_t *__restrict__ ids,
@@ -508,11 +510,13 @@ int dispatch_launch(const uint32_t *ids, uint64_t tokens, uint32_t top_k, uint32
         // reads them, so the buffer needs no clearing between calls.
         bc = bc_ws;
     }
-    // Sixteen wavefronts a block place a quarter of the assignments each that
-    // four do, one dependent round of 64 after another; their cursors have to
-    // fit the LDS (72 KB at 1024 experts), and up to 512 assignments are two
-    // rounds for four.  Both launches, 131072 assignments: 14.4 -> 11.9 us at
-    // 128 experts, 19.2 -> 13.2 at 256.
+    // Sixteen wavefronts a block where the counts that every block reads are
+    // many (their cursors have to fit the LDS: 72 KB at 1024 experts): 131072
+    // assignments 14.2 -> 11.6 us at 128 experts (8192 counts), 19.1 -> 13.0 at
+    // 256; 8000 at 1024 (4096 counts) 14.3 -> 13.0; 24000 at 256 (3072) 11.9 ->
+    // 11.2.  Below, the larger workgroup costs about what it gains or more: 600
+    // assignments at 8 experts 4.2 -> 5.5, 2400 at 128 8.5 -> 9.8, 98304 at 8
+    // 9.3 -> 9.9.
     auto launch = [&]<uint32_t BLOCK>() {
         if (bc)
             FELLM_LAUNCH((moe_count_blocks<BLOCK>), dim3(g.nblocks), dim3(BLOCK), (size_t)E * sizeof(uint32_t), st, ids, n,
@@ -521,7 +525,7 @@ int dispatch_launch(const uint32_t *ids, uint64_t tokens, uint32_t top_k, uint32
         FELLM_LAUNCH((moe_scatter_blocks<BLOCK>), dim3(g.nblocks), dim3(BLOCK), lds, st, ids, n, E, bits, g.chunk,
                      g.nblocks, bc, counts, offsets, order, inv, err_flag);
     };
-    if (n > 512 && E <= 1024)
+    if (g.nblocks * E >= 3072 && E <= 1024)
         launch.template operator()<1024>();
     else
         launch.template operator()<256>();
@@ -600,7 +604,7 @@ extern "C" int fellm_rocm_moe_gather(const void *x, uint32_t elem_bytes, uint64_
     if (inv && vec16) {
         const uint64_t row_vecs = row_bytes / 16;
         const uint32_t grid = grid_cap(tokens, 16384);
-        const bool nt = n * row_bytes >= kStreamBytes;
+        const bool nt = n * row_bytes >= kGatherStreamBytes;
 #define FELLM_MOE_SCATTER(SEG, NT)                                                                                  \
     FELLM_LAUNCH((moe_scatter_rows<SEG, NT>), dim3(grid), dim3(256), 0, st, static_cast<const uint4 *>(x), order, \
                        inv, tokens, top_k, row_vecs, static_cast<uint4 *>(grouped))
@@ -641,13 +645,13 @@ extern "C" int fellm_rocm_moe_combine(const float *y0, const float *expert_out, 
     hipStream_t st = as_stream(stream);
     const uint32_t grid = grid_cap(tokens, 65536);
     const bool vec = hidden % 4 == 0 && aligned_to(expert_out, 16) && aligned_to(y, 16) && (!y0 || aligned_to(y0, 16));
-    const uint32_t block = hidden / (vec ? 4 : 1) > 512 ? 1024 : 512;
-    const bool nt = n * hidden * sizeof(float) >= kStreamBytes;
+    const bool nt = vec && n * hidden * sizeof(float) >= kCombineStreamBytes;
+    const uint32_t block = hidden / (vec ? 4 : 1) > 512 && (nt || tokens <= 2ull * cu_count()) ? 1024 : 512;
 #define FELLM_MOE_COMBINE(ORD, V, NT)                                                                              \
     FELLM_LAUNCH((moe_combine_rows<ORD, V, NT>), dim3(grid), dim3(block), 0, st, y0, expert_out, ids, weights, inv, \
                        tokens, top_k, hidden, n, y)
 #define FELLM_MOE_COMBINE_V(ORD)          \
-    if (vec && nt)                        \
+    if (nt)                               \
         FELLM_MOE_COMBINE(ORD, 4, true);  \
     else if (vec)                         \
         FELLM_MOE_COMBINE(ORD, 4, false); \

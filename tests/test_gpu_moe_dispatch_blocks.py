@@ -1,6 +1,6 @@
-"""MoE dispatch around the choice of its workgroup (1024 threads from 513
-assignments on, up to 1024 experts) and around the chunks and rounds of its
-sixteen wavefronts; exact against the oracle."""
+"""MoE dispatch around the choice of its workgroup (1024 threads where blocks x
+experts reach 3072, up to 1024 experts) and around the chunks and rounds of its
+four or sixteen wavefronts; exact against the oracle."""
 from __future__ import annotations
 
 import numpy as np
@@ -22,3 +22,9 @@ def test_dispatch_blocks(tokens, k, n_experts):
     d = ops.moe_dispatch(torch.from_numpy(ids.view(np.int32)).cuda(), n_experts)
     for got, want in zip(d, oracle.moe_dispatch(ids, n_experts)):
         assert np.array_equal(got.cpu().numpy().view(np.uint32), want)
+
+
+@pytest.mark.parametrize("tokens,k,n_experts", [(4096, 1, 1024), (4097, 1, 1024), (6145, 1, 1025), (47104, 1, 128),
+                                                (47105, 1, 128), (6000, 8, 127), (24700, 8, 16)])
+def test_dispatch_workgroup_choice(tokens, k, n_experts):
+    test_dispatch_blocks(tokens, k, n_experts)

@@ -1,6 +1,6 @@
 """MoE gather and combine above the size from which their rows are streamed
-(128 MiB of expert or grouped rows) and below it, at row lengths around the
-combine's 512- and 1024-thread workgroups; bit-exact against torch on the same
+(128 MiB of grouped, 192 MiB of expert rows) and below it, at row lengths and
+token counts around the combine's 512- and 1024-thread workgroups; bit-exact against torch on the same
 rows (the combine's adds in order, each product rounded before its sum)."""
 from __future__ import annotations
 
@@ -21,9 +21,12 @@ def _ids(gen, tokens, k, n_experts):
     return torch.argsort(torch.rand(tokens, n_experts, generator=gen, device="cuda"), 1)[:, :k].to(torch.int32).contiguous()
 
 
-# expert rows: 139 MB, 135 MB, 134.2 MB (the limit itself), 134.2 MB less a row, 4 MB
+# expert rows: 139 MB, 135 MB, 134.2 MB, 134.2 MB less a row, 4 MB; 204 MB, 202 MB, 201.3 MB (the limit itself),
+# 201.3 MB less a row; more than 512 vectors or elements a row for 512 tokens and 513
 @pytest.mark.parametrize("tokens,k,hidden", [(1500, 8, 2892), (16500, 8, 256), (8192, 2, 2048), (8191, 2, 2048),
-                                             (65, 8, 2048)])
+                                             (65, 8, 2048), (2200, 8, 2892), (24600, 8, 256), (12288, 2, 2048),
+                                             (12287, 2, 2048), (512, 4, 2052), (513, 4, 2052), (512, 2, 1001),
+                                             (513, 2, 1001)])
 def test_combine_streamed(ops, tokens, k, hidden):
     gen = torch.Generator(device="cuda").manual_seed(tokens)
     ids = _ids(gen, tokens, k, 32)

@@ -99,6 +99,14 @@ def test_dense_f32_gather_and_norm(ops, dim, n):
     assert np.abs(y.cpu().numpy() - ref).max() <= 1e-5 * np.abs(ref).max()
 
 
+@pytest.mark.parametrize("n", [3, 512, 513])
+@pytest.mark.parametrize("dim", [4096, 4100, 8196, 16380])
+def test_dense_f32_gather_parts(ops, dim, n):
+    """Rows of an odd number of 4-element parts beside even ones, on both sides
+    of the row count that chooses between parts of 8 and of 4."""
+    test_dense_f32_gather_and_norm(ops, dim, n)
+
+
 def test_bf16_gather_keeps_nan_payloads(ops):
     rng = np.random.default_rng(9)
     table = rng.integers(0, 1 << 16, size=(64, 512), dtype=np.uint32).astype(np.uint16)  # every kind of bf16

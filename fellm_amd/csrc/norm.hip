@@ -322,6 +322,9 @@ int launch_typed(const void *x, const void *r, void *h, const float *w, void *y,
     if (vec_ok) {
         // Few rows (decode): wide blocks keep more bytes in flight per CU.
         if (rows < 1024 && group <= 1024 * 8 * 2) {
+            // f32 rows with threads to spare, one chunk each: 1023 rows of 64
+            // without a residual 4.16 -> 3.84 us (but of 4096 7.1 -> 8.4).
+            if (M > 1 && group <= 1024) return launch_fast<A, O, 1024, VEC, 1>(x, r, h, w, y, group, rows, eps, s);
             if (group <= 1024 * 8) return launch_fast<A, O, 1024, VEC, M>(x, r, h, w, y, group, rows, eps, s);
             return launch_fast<A, O, 1024, VEC, 2 * M>(x, r, h, w, y, group, rows, eps, s);
         }

@@ -266,39 +266,20 @@ __device__ __forceinline__ uint4 lds_u4(const void *p) { return *reinterpret_cas
 // Cache policy 2 = non-temporal (read once).
 using Rsrc = __amdgpu_buffer_rsrc_t;
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
-typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 __device__ __forceinline__ Rsrc weight_rsrc(const uint8_t *w, uint32_t bytes) {
     return __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t *>(w), 0, (int)bytes, 0x00020000);
 }
-__device__ __forceinline__ uint4 bld16(Rsrc r, uint32_t off) {
-    const u32x4 v = __builtin_amdgcn_raw_buffer_load_b128(r, off, 0, 2);
-    return make_uint4(v.x, v.y, v.z, v.w);
-}
-__device__ __forceinline__ uint2 bld8(Rsrc r, uint32_t off) {
-    const u32x2 v = __builtin_amdgcn_raw_buffer_load_b64(r, off, 0, 2);
-    return make_uint2(v.x, v.y);
-}
-__device__ __forceinline__ uint32_t bld2(Rsrc r, uint32_t off) {
-    return __builtin_amdgcn_raw_buffer_load_b16(r, off, 0, 2);
-}
-
 __device__ __forceinline__ float f16_bits(uint32_t b) { return (float)__builtin_bit_cast(_Float16, (uint16_t)b); }
-
-__device__ __forceinline__ uint32_t bld4(Rsrc r, uint32_t off) {
-    return __builtin_amdgcn_raw_buffer_load_b32(r, off, 0, 2);
-}
 
 // Partner lane of a pair (lane ^ 1): DPP quad_perm [1,0,3,2].
 __device__ __forceinline__ uint32_t pair_swap(uint32_t v) { return dpp_u32<0xB1>(v); }
-
-__device__ __forceinline__ uint32_t mask_shr(uint32_t v, uint32_t s, uint32_t m) { return (v >> s) & m; }
 
 // ---- lane layout ----------------------------------------------------------------
 // Two lanes per 256-element block: lane half h (= lane & 1) covers elements
 // 128h .. 128h+127.  The 32 lane pairs of a wavefront take 32 block slots:
 // with nb <= 32 blocks per row, slot s is block s % nb of row s / nb of the
-// wavefront's current row group (32 / nb rows at once); with nb > 32 a row is
-// walked in passes of 32 blocks.  Bytes both lanes of a block need (the
+// wavefront's current row group (32 / nb rows at once); with nb > 32 it is
+// block s of the wavefront's share of a row.  Bytes both lanes of a block need (the
 // Q4_K/Q5_K header, the Q5_K high bits) are loaded half by each lane and
 // exchanged with one DPP swap: lanes reading the same address in one load
 // slow the memory pipeline measurably.
@@ -530,7 +511,7 @@ __device__ __forceinline__ float fold_serial(const float *f, uint32_t n, float a
 
 // ---- staging: coalesced 16-byte loads of a contiguous byte range ---------------
 // A wavefront's unit of work is a contiguous byte range of each matrix (a
-// group of whole rows, or one 32-block pass of a row) of at most 32 blocks.
+// group of whole rows, or its share of a longer row) of at most 32 blocks.
 // It is fetched as aligned 16-byte chunks, lane l taking chunk 64i + l, so
 // one load instruction covers 1 KB of consecutive bytes (the pattern that
 // reaches the copy-kernel bandwidth; per-block lane patterns measured
@@ -569,7 +550,7 @@ constexpr uint32_t kStagePerWave = 1024 * (kChunks<GW> + (FUSED ? kChunks<UW> : 
 // lane pair slot s works on block s % nb of row s / nb; the lane's x slice
 // stays in registers for the whole launch.
 // Each step: next unit's loads issued -> block values of the staged unit ->
-// fold buffer; after a row's last unit, lanes 0 .. mats*rows-1 each fold one
+// fold buffer, from which lanes 0 .. mats*rows-1 each fold one
 // (row, matrix) serially over its block values from 0.0 and the even lanes
 // apply silu(gate) * up; then the next unit is written to the stage.
 template <typename GW, typename UW, bool FUSED, bool PREQ, int NW = kGemvWaves>
@@ -858,7 +839,7 @@ __global__ __launch_bounds__(kGemvBlock) void quantize_q8k_kernel(const float *_
     quantize_x(x, nb, xl, blockIdx.x * kGemvWaves + threadIdx.x / kWave, gridDim.x * kGemvWaves);
 }
 
-// Workgroups for `units` row groups (or rows of passes).  Each workgroup
+// Workgroups for `units` row groups of at most 32 blocks.  Each workgroup
 // quantizes x once, so a launch keeps to FELLM_GEMV_MAX_GRID (512) unless
 // its wavefronts would each get more than two units; then it widens to at
 // most FELLM_GEMV_WIDE_GRID (768), and never past the workgroups that can be

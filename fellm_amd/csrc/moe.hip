@@ -308,11 +308,17 @@ __device__ __forceinline__ void store_vec(V *p, const V &v) {
 }
 
 // Bytes from which the grouped rows (gather) and the expert rows (combine) are
-// streamed: half and three quarters of the 256 MB last-level cache.  Below, a
-// caller's next or previous kernel may find them there.  Measured: gather of
-// 134 MB 37.7 -> 30.7 us; combine of 240 MB 64.3 -> 56.3 us, of 180 MB 47.2 ->
-// 48.7, of 134 MB 39.6 -> 41.9.
-constexpr uint64_t kGatherStreamBytes = 128ull << 20, kCombineStreamBytes = 192ull << 20;
+// streamed, around the 256 MB of the last-level cache: below, a caller's next
+// or previous kernel may find them there.  Gather rows of more than 4 KB from
+// half of it (189 MB in rows of 5760 bytes 65 -> 43 us, with a pass over them
+// 120 -> 108), shorter ones from all of it (268 MB in rows of 2 KB 56 -> 52 and
+// 149 -> 144; 201 MB in rows of 1536 bytes 36 -> 39 and 98 -> 109), and only whole
+// cache lines, since a streamed store writes parts of lines at once (262 MB in
+// rows of 2000 bytes 63 -> 71 us).  Combine: 240 MB 64.3 -> 56.3 us, 180 MB
+// 47.2 -> 48.7, 134 MB 39.6 -> 41.9.
+constexpr uint64_t kGatherStreamBytes = 128ull << 20, kGatherStreamBytesShort = 256ull << 20;
+constexpr uint64_t kCombineStreamBytes = 192ull << 20;
+constexpr uint32_t kLineBytes = 128;
 
 // grouped[i] = x[order[i] / top_k]; an invalid order entry gives a zero row.
 template <typename V>
@@ -604,7 +610,8 @@ extern "C" int fellm_rocm_moe_gather(const void *x, uint32_t elem_bytes, uint64_
     if (inv && vec16) {
         const uint64_t row_vecs = row_bytes / 16;
         const uint32_t grid = grid_cap(tokens, 16384);
-        const bool nt = n * row_bytes >= kGatherStreamBytes;
+        const bool nt = n * row_bytes >= (row_vecs <= 256 ? kGatherStreamBytesShort : kGatherStreamBytes) &&
+                        row_bytes % kLineBytes == 0 && aligned_to(grouped, kLineBytes);
 #define FELLM_MOE_SCATTER(SEG, NT)                                                                                  \
     FELLM_LAUNCH((moe_scatter_rows<SEG, NT>), dim3(grid), dim3(256), 0, st, static_cast<const uint4 *>(x), order, \
                        inv, tokens, top_k, row_vecs, static_cast<uint4 *>(grouped))

@@ -1,5 +1,5 @@
 """MoE gather and combine above the size from which their rows are streamed
-(128 MiB of grouped, 192 MiB of expert rows) and below it, at row lengths and
+(128 or 256 MiB of grouped rows by their length, 192 MiB of expert rows) and below it, at row lengths and
 token counts around the combine's 512- and 1024-thread workgroups; bit-exact against torch on the same
 rows (the combine's adds in order, each product rounded before its sum)."""
 from __future__ import annotations
@@ -48,8 +48,10 @@ def test_combine_streamed(ops, tokens, k, hidden):
     assert torch.equal(in_place, want_e)
 
 
-# grouped rows: 135 MB in one and in several segments per thread, 2 MB
-@pytest.mark.parametrize("tokens,k,hidden", [(16500, 2, 2048), (2000, 8, 4224), (65, 8, 2048)])
+# grouped rows: 135 MB in one and in several segments per thread, 2 MB; 270 MB in one segment, 135 MB and 269 MB in
+# rows that end inside a cache line
+@pytest.mark.parametrize("tokens,k,hidden", [(16500, 2, 2048), (2000, 8, 4224), (65, 8, 2048), (16500, 4, 2048),
+                                             (2000, 8, 4232), (16500, 4, 2040)])
 def test_gather_streamed(ops, tokens, k, hidden):
     gen = torch.Generator(device="cuda").manual_seed(hidden)
     ids = _ids(gen, tokens, k, 16)

@@ -71,7 +71,6 @@ struct F32kvArgs {
     // 2: keys within `window` of the row index (all when window == 0).
     uint32_t row_mode, window;
     uint32_t head_major;  // q and out are [head][row][d] instead of [row][head][d]
-    uint32_t out_vec;     // out is 16-byte aligned
 };
 
 // Keys [lo, hi) of the first pair that query row `row` attends.
@@ -369,13 +368,11 @@ __global__ __launch_bounds__(NW *kWave) void attention_f32kv_kernel(F32kvArgs a)
                 float r[VW];
 #pragma unroll
                 for (int x = 0; x < VW; ++x) r[x] = l > 0.0f ? acc[h * VW + x][e] * inv : 0.0f;
+                // Element stores, which become one vector store of any 4-byte
+                // alignment; a branch on out's alignment made two of each.
                 if (FULL || d < hd) {
-                    if (a.out_vec) {
-                        store_f32<F32, VW>(a.out + qoff + d, r);
-                    } else {
 #pragma unroll
-                        for (int x = 0; x < VW; ++x) a.out[qoff + d + x] = r[x];
-                    }
+                    for (int x = 0; x < VW; ++x) a.out[qoff + d + x] = r[x];
                 }
             }
     }
@@ -425,7 +422,7 @@ int attention_f32kv_common(const float *q, float *out, uint32_t rows, uint32_t n
     if (rows == 0) return FELLM_OK;
     if (!(scale > 0.0f)) scale = 1.0f / sqrtf((float)head_dim);
     F32kvArgs a{q, out, k1, v1, k2, v2, rows, n_heads, n_kv_heads, head_dim, begin1, end1, n2, scale, row_mode,
-                window, head_major, aligned_to(out, 16)};
+                window, head_major};
     hipStream_t st = as_stream(stream);
     if (head_dim <= 64) return choose_f32kv<64>(a, st);
     if (head_dim <= 128) return choose_f32kv<128>(a, st);

@@ -11,8 +11,8 @@
 //   :138-174 address them.
 //
 // Work split.  One workgroup per (key split s, batch row b, KV head g), its
-// four wavefronts taking every fourth pair of cache blocks and merging their
-// (max, sum, accumulators) through LDS at the end; the
+// four wavefronts (or one: one_wave below) taking every fourth pair of cache
+// blocks and merging their (max, sum, accumulators) through LDS at the end; the
 // G = n_heads / n_kv query heads that share KV head g are processed together
 // (as up to 16 head slots), so every K/V byte is read once.  Both products of a
 // pair of blocks (2 x 16 tokens) run on the matrix cores:
@@ -41,7 +41,7 @@
 // Bound by the cache's bytes.  Against the kernel before it (one wavefront per
 // workgroup, P.V on the vector ALUs, two blocks ahead): 256 rows of 256 .. 4096
 // keys, 64/8 heads of 128, bf16 (2.39 GB) 629 -> 414 us; the same of 4096 keys
-// each 747 -> 709 (6.1 TB/s); one row of 32768 keys, 32/8 heads, f16 33.9 -> 27.3.
+// each 747 -> 709 (6.1 TB/s); one row of 32768 keys, 32/8 heads, f16 33.9 -> 27.6.
 //
 // Splits write unnormalised partial sums with their running max and
 // denominator; a second kernel combines them.  A row whose keys fit one split
@@ -67,7 +67,7 @@ constexpr uint32_t kBlockTokens = 16;  // tokens per cache block handled by one 
 // floats, so that every record starts on a 16-byte boundary.
 constexpr uint32_t kRecTail = 4;
 // Wavefronts that share a split's blocks.  Measured (kernels of 1 / 2 / 4 / 8,
-// f16): 256 rows of 256 .. 4096 keys 445 / 416 / 396 / 462 us, one row of 32768
+// f16, two parts of p): 256 rows of 256 .. 4096 keys 445 / 416 / 396 / 462 us, one row of 32768
 // keys 31.6 / 26.3 / 27.3 / 31.0, 256 rows of 16 .. 256 keys 36 / 30 / 36 / 67.
 constexpr uint32_t kDecodeWaves = 4;
 // Cache policies of the K and V reads.  V is read once by whole lines, so it

@@ -288,8 +288,8 @@ int fellm_rocm_paged_attention(const void *q, uint32_t q_dtype, void *out, uint3
  * 1/sqrt(head_dim); query head h uses KV head h / (n_heads / n_kv_heads).
  * No keys gives a zero row.  head_dim % 4 == 0, head_dim <= 256,
  * (n_heads / n_kv_heads) * head_dim <= 2048; q, k1, v1, k2 and v2 16-byte
- * aligned, out 4-byte.  out may be q itself
- * and must not overlap q otherwise, nor k1, v1, k2 or v2.
+ * aligned, out 4-byte.  out may be q itself and must not overlap q otherwise,
+ * nor k1, v1, k2 or v2.
  * Accumulation and the softmax run in f32 with the device exp.
  */
 int fellm_rocm_attention_f32kv(const float *q, float *out, uint32_t rows, uint32_t n_heads, uint32_t n_kv_heads,
